@@ -327,7 +327,7 @@ struct ssg_registration {
   // batch workspace
   int cap = 0;
   DevBuf cur_pyr, cur_mask_pyr, half_buf, norm_buf, gray_buf;
-  DevBuf xf_t, xf_m, res, partials, active[2], active_count[2], lm;
+  DevBuf xf_t, xf_m, res, partials, active[2], active_count[2], lm, memo;
   DevBuf frame_ptrs, mask_ptrs, zero_count, frame_list, tmp_in, tmp_mask, sum_tmp;
   DevBuf half_ptrs;  // sources of the batched half-size pyrDown
   int* pinned_count = nullptr;
@@ -614,6 +614,7 @@ int ensure_workspace(ssg_registration* r, int n) {
   CHK(r->res.ensure(sizeof(FrameRes) * n));
   CHK(r->partials.ensure(sizeof(double) * (size_t)n * tx0 * ty0 * NMOM_FULL));
   if (r->o.ecc.ecc_method != SSG_ECC_ALIGN_FORWARD_ADDITIVE) CHK(r->lm.ensure(sizeof(FrameLm) * n));
+  else CHK(r->memo.ensure(sizeof(EccMemo) * n));
   for (int i = 0; i < 2; ++i) {
     CHK(r->active[i].ensure(sizeof(int) * n));
     CHK(r->active_count[i].ensure(sizeof(int) * 4));
@@ -664,9 +665,11 @@ int run_ecc(ssg_registration* r, int n, int pass, bool has_cmask, bool plain, bo
     // the inverse-compositional J is dropped whenever the translation-first pass swaps
     // the aligner's transform (c_frame_registration.cc:823,844); otherwise it persists
     lb.jrec = (method == ECC_IC || method == ECC_ICLM) && !tfirst ? r->jrec.as<JRec>() : nullptr;
+    lb.memo = method == ECC_FA && motion == SSG_MOTION_TRANSLATION ? r->memo.as<EccMemo>() : nullptr;
     HIPCHK(launch_level_begin(lb, s));
 
     EccPassArgs a{};
+    a.memo = r->memo.as<EccMemo>();
     a.cur = r->cur_pyr.as<float>() + r->loff[l];
     a.cur_fstride = r->pyr_elems;
     a.cur_pitch = r->lpitch[l];

@@ -72,6 +72,19 @@ constexpr int NMOM_LM_TRANS = 6;  // gx^2, gx gy, gy^2, gx rhs, gy rhs, |rhs|^2
 constexpr int NMOM_IC = 8;        // inverse-compositional pass: 6 J^T rhs moments, |rhs|^2, good pixels
 constexpr int NMOM_REF = 18;      // reference-gradient Hessian moments of a level
 
+// The moments of a translation pass depend on the translation only through the quantised sample
+// positions (1/32 px, the same for every pixel) and on the centring constant: a frame that steps back
+// to a quantised position it was at in this level with the same constant has its moments here and needs
+// no pass over the image.  The 1/32-px steps are coarser than the stopping threshold, so near the optimum the aligner
+// walks between a few neighbouring positions until its budget is spent.
+constexpr int ECC_MEMO = 64;
+struct EccMemo {
+  int count;  // moments stored in this level; entry count % ECC_MEMO is written next
+  int qx[ECC_MEMO], qy[ECC_MEMO];
+  float cg[ECC_MEMO];
+  double G[ECC_MEMO][NMOM_TRANS];
+};
+
 constexpr int ECC_LW = 64;                    // LDS row width: one column per lane
 constexpr int ECC_TW = ECC_LW - 4;            // output columns per tile (2-px gradient halo each side)
 constexpr int ECC_RPT = 16;                   // rows per thread
@@ -116,6 +129,7 @@ struct EccPassArgs {
   int max_iterations;
   float max_eps;
   double update_step_scale;
+  EccMemo* memo;          // per frame, forward-additive translation passes
   // Levenberg-Marquardt / inverse-compositional aligners
   int method;              // ECC_*
   FrameLm* lm;
@@ -162,6 +176,7 @@ struct LevelBeginArgs {
   int method;              // ECC_*
   FrameLm* lm;
   JRec* jrec;              // per-level record when J persists across frames, else null
+  EccMemo* memo;           // emptied at the level start (translation passes), or null
 };
 
 // ---- input stage (raw frames -> pipeline f32 images, debayer) ----------------------------------

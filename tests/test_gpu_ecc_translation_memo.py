@@ -1,0 +1,65 @@
+"""Translation iterations that step back to a quantised position they were at: the moments kept from
+the first visit must give the step a pass over the image gives, and the rule that says when a
+translation quantises alike for every pixel must hold."""
+import numpy as np
+import pytest
+
+from tests import synth_np
+
+
+@pytest.mark.parametrize("n", [16, 61, 1920, 4096, 8192])
+def test_key_rule_quantises_every_pixel_alike(n):
+    """fl(fl(x + t) * 32) rounds to 32 x + rint(32 t) for every pixel x whenever 32 t is farther from a
+    rounding tie than (n + |t| + 2) 2^-18 (the device's rule, restated in float32)."""
+    rng = np.random.default_rng(n)
+    x = np.arange(n, dtype=np.float32)
+    t = rng.uniform(-40, 40, 400).astype(np.float32)
+    ties = (rng.integers(-900, 900, 400) + 0.5) / 32  # and translations a few steps beside a tie
+    t = np.concatenate([t, (ties + rng.normal(0, 1, 400) * n * 2.0 ** -24).astype(np.float32),
+                        np.float32([0.0, 1.0, -1.0, 1 / 64, -1 / 64, 0.015625 + 1e-6])])
+    seen = 0
+    for v in t:
+        u = np.float32(32) * v
+        r = np.rint(u)
+        if not abs(u - r) < np.float32(0.5) - (np.float32(n) + abs(v) + np.float32(2)) * np.float32(2.0 ** -18):
+            continue
+        seen += 1
+        q = np.rint((x + v) * np.float32(32)).astype(np.int64)
+        assert np.array_equal(q, 32 * x.astype(np.int64) + int(r)), v
+    assert seen > 300
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("w,h", [(61, 65), (120, 64), (333, 241)])
+def test_every_step_is_the_step_of_its_position(oracle64, w, h):
+    """The positions after budgets of 1 .. 40 iterations (a threshold that is never met, so the aligner
+    walks between neighbouring positions): each next one is one FP64 oracle step from the last.  32-bit
+    sums of about 30 roundings (2e-6 of the sum of magnitudes, which is a few pixels of step at the most)
+    leave 1e-4 px."""
+    import serstacker_amd as S
+    import torch
+
+    ref, frames, _ = synth_np.frames(3, w, h, radius=0.4 * min(w, h), seed=w, shift=2.0, rot_deg=0.3, noise=0.004)
+    dev = [torch.from_numpy(np.ascontiguousarray(f)).cuda() for f in frames]
+    path = [np.zeros((3, 2), np.float32)]
+    for k in range(1, 41):
+        reg = S.c_frame_registration(S.c_image_registration_options(
+            motion_type=0, scale=1.0, eps=1e-7, ecch_max_level=1, max_iterations=k, input_smooth_sigma=0.0,
+            reference_smooth_sigma=0.0, min_rho=0.0))
+        assert reg.setup_reference_frame(np.ascontiguousarray(ref, dtype=np.float32))
+        st = reg.register_batch(dev)
+        assert all(s.iterations == k + 1 for s in st)
+        path.append(np.array([[s.params[0], s.params[1]] for s in st], np.float32))
+    revisits = 0
+    for f in range(3):
+        seen = set()
+        for k in range(40):
+            p, u = path[k][f], path[k][f].astype(np.float64) * 32
+            revisits += tuple(np.rint(u)) in seen
+            seen.add(tuple(np.rint(u)))
+            if np.abs(np.abs(u - np.rint(u)) - 0.5).min() < (max(w, h) + 4) * 2.0 ** -18:
+                continue  # the oracle's exact sum may round to the other side
+            t = oracle64.xform(0, [float(p[0]), float(p[1])])
+            oracle64.ecc_fa_align(ref.astype(np.float32), frames[f], t, max_iterations=1, max_eps=1e-7)
+            assert np.abs(np.array(t.p[:2]) - path[k + 1][f]).max() < 1e-4, (f, k)
+    assert revisits > 20
