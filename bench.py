@@ -888,7 +888,7 @@ def bench_sweep(a, S, _lib, torch):
     pc = S.phase_correlation(W, H, 2)
     pc.set_reference(raw[0])
     M = 2048 * 2048
-    timed("phasecorr_64x4096x3000_binned2", lambda: pc.estimate(views), n * (2 * W * H + 17 * 8 * M), n, "frames")
+    timed("phasecorr_64x4096x3000_binned2", lambda: pc.estimate(views), n * (2 * 2 * W * H + 3 * 8 * M), n, "frames")
     del raw, views
     # focus stacking: 16 RGB f32 frames of 2048x1536 per stack (add + compute)
     W, H, n = 2048, 1536, 16

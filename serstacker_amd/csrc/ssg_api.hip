@@ -2918,7 +2918,7 @@ extern "C" int ssg_accumulation_get_profile(ssg_accumulation* a, ssg_profile* ou
 struct ssg_phasecorr {
   int w = 0, h = 0, binning = 1, bw = 0, bh = 0, M = 0, N = 0;
   hipStream_t stream = nullptr;
-  DevBuf wx, wy, tw_m, tw_n, ref_spec, buf, tmp, frame_ptrs, out, mean, part, pv, pi;
+  DevBuf wx, wy, tw_m, tw_n, ref_spec, plane, frame_ptrs, out, mean, part, pv, pi;
   int chunk = 1;
   bool have_ref = false;
   Profiler prof;
@@ -2937,15 +2937,29 @@ int pow2_at_least(int n) {
   return p;
 }
 
-// frames -> spectra in pc->tmp ([M][N] per frame)
-int pc_spectra(ssg_phasecorr* pc, int n, const void* const* dev_ptrs, bool u16, int pitch) {
-  hipStream_t s = pc->stream;
+// two binned pixels' samples per load: every frame's rows start at a multiple of their bytes
+bool pc_wide(const ssg_phasecorr* pc, int n, const void* const* ptrs, size_t step, int es) {
+  const size_t unit = (size_t)2 * pc->binning * es;
+  if (step % unit) return false;
+  for (int f = 0; f < n; ++f)
+    if ((uintptr_t)ptrs[f] % unit) return false;
+  return true;
+}
+
+// means of n frames
+int pc_means(ssg_phasecorr* pc, int n, const void* const* dev_ptrs, bool u16, int pitch, bool wide) {
   CHK(pc->mean.ensure(sizeof(float) * n));
   CHK(pc->part.ensure(sizeof(double) * PC_PARTS_MAX * n));
-  HIPCHK(launch_pc_load(dev_ptrs, u16, pitch, pc->bw, pc->bh, pc->binning, pc->mean.as<float>(), pc->part.as<double>(),
-                        pc->wx.as<float>(), pc->wy.as<float>(), pc->buf.as<float2>(), pc->M, pc->N, n, s));
-  HIPCHK(launch_fft2(pc->buf.as<float2>(), pc->tmp.as<float2>(), pc->M, pc->N, n, pc->tw_m.as<float2>(),
-                     pc->tw_n.as<float2>(), false, s));
+  HIPCHK(launch_pc_mean(dev_ptrs, u16, pitch, wide, pc->bw, pc->bh, pc->binning, pc->mean.as<float>(),
+                        pc->part.as<double>(), n, pc->stream));
+  return SSG_OK;
+}
+
+// row transforms of n frames from f0 on into pc->plane
+int pc_rows(ssg_phasecorr* pc, int f0, int n, const void* const* dev_ptrs, bool u16, int pitch, bool wide) {
+  HIPCHK(launch_pc_rows(dev_ptrs + f0, u16, pitch, wide, pc->bw, pc->bh, pc->binning, pc->mean.as<float>() + f0,
+                        pc->wx.as<float>(), pc->wy.as<float>(), pc->tw_m.as<float2>(), pc->plane.as<float2>(), pc->M,
+                        pc->N, n, pc->stream));
   return SSG_OK;
 }
 }  // namespace
@@ -2984,9 +2998,10 @@ extern "C" int ssg_phasecorr_create(int32_t width, int32_t height, int32_t binni
   HIPCHK(hipMemcpyAsync(pc->wy.p, wy.data(), sizeof(float) * wy.size(), hipMemcpyHostToDevice, pc->stream));
   HIPCHK(hipMemcpyAsync(pc->tw_m.p, tm.data(), sizeof(float2) * tm.size(), hipMemcpyHostToDevice, pc->stream));
   HIPCHK(hipMemcpyAsync(pc->tw_n.p, tn.data(), sizeof(float2) * tn.size(), hipMemcpyHostToDevice, pc->stream));
-  // frames per launch: two complex planes per frame, at most about 2 GiB in flight
-  const size_t per = (size_t)pc->M * pc->N * sizeof(float2);
-  pc->chunk = (int)std::max<size_t>(1, std::min<size_t>(64, ((size_t)2 << 30) / (2 * per)));
+  // frames per launch: planes of 512 MB in all (16 padded 2048 x 2048 frames; 128 MB was 20 % slower, 2 GB
+  // 2 % faster)
+  const size_t per = pc_plane(pc->M, pc->N) * sizeof(float2);
+  pc->chunk = (int)std::max<size_t>(1, std::min<size_t>(64, ((size_t)512 << 20) / per));
   CHK(pc->ref_spec.ensure(per));
   HIPCHK(hipStreamSynchronize(pc->stream));
   *out = pc.release();
@@ -3006,14 +3021,16 @@ extern "C" int ssg_phasecorr_set_reference(ssg_phasecorr* pc, const ssg_image* r
   const void* p;
   size_t pb;
   CHK(device_view(ref, t, s, &p, &pb));
-  const size_t per = (size_t)pc->M * pc->N * sizeof(float2);
-  CHK(pc->buf.ensure(per));
-  CHK(pc->tmp.ensure(per));
+  CHK(pc->plane.ensure(pc_plane(pc->M, pc->N) * sizeof(float2)));
   CHK(pc->frame_ptrs.ensure(sizeof(void*)));
   HIPCHK(hipMemcpyAsync(pc->frame_ptrs.p, &p, sizeof(void*), hipMemcpyHostToDevice, s));
   const bool u16 = ref->type == SSG_16UC1;
-  CHK(pc_spectra(pc, 1, pc->frame_ptrs.as<const void*>(), u16, (int)(pb / (u16 ? 2 : 4))));
-  HIPCHK(hipMemcpyAsync(pc->ref_spec.p, pc->tmp.p, per, hipMemcpyDeviceToDevice, s));
+  const int es = u16 ? 2 : 4;
+  const bool wide = pc_wide(pc, 1, &p, pb, es);
+  CHK(pc_means(pc, 1, pc->frame_ptrs.as<const void*>(), u16, (int)(pb / es), wide));
+  CHK(pc_rows(pc, 0, 1, pc->frame_ptrs.as<const void*>(), u16, (int)(pb / es), wide));
+  HIPCHK(launch_pc_cols(pc->plane.as<float2>(), pc->ref_spec.as<float2>(), pc->tw_n.as<float2>(), pc->M, pc->N,
+                        pc->bh, true, 1, s));
   HIPCHK(hipStreamSynchronize(s));
   pc->have_ref = true;
   return SSG_OK;
@@ -3037,35 +3054,35 @@ extern "C" int ssg_phasecorr_estimate(ssg_phasecorr* pc, int n, const ssg_image*
   }
   if (frames[0].step % es) return fail(SSG_E_INVALID_ARG, "frame step must be a multiple of the element size");
   hipStream_t s = pc->stream;
-  const int chunk = std::min(pc->chunk, n);
+  const int chunks = (n + pc->chunk - 1) / pc->chunk, chunk = (n + chunks - 1) / chunks;  // of even size
   const long long per = (long long)pc->M * pc->N;
-  CHK(pc->buf.ensure(sizeof(float2) * per * chunk));
-  CHK(pc->tmp.ensure(sizeof(float2) * per * chunk));
+  const int groups = pc_groups(pc->M, pc->N);
+  CHK(pc->plane.ensure(sizeof(float2) * pc_plane(pc->M, pc->N) * chunk));
+  CHK(pc->pv.ensure(sizeof(float) * (size_t)groups * chunk));
+  CHK(pc->pi.ensure(sizeof(int) * (size_t)groups * chunk));
   CHK(pc->frame_ptrs.ensure(sizeof(void*) * n));
   CHK(pc->out.ensure(sizeof(double) * 3 * n));
   std::vector<const void*> ptrs(n);
   for (int f = 0; f < n; ++f) ptrs[f] = frames[f].data;
   HIPCHK(hipMemcpyAsync(pc->frame_ptrs.p, ptrs.data(), sizeof(void*) * n, hipMemcpyHostToDevice, s));
   const int pitch = (int)(frames[0].step / es);
+  const bool wide = pc_wide(pc, n, ptrs.data(), (size_t)frames[0].step, es);
   pc->prof.start(s);
+  CHK(pc_means(pc, n, pc->frame_ptrs.as<const void*>(), type == SSG_16UC1, pitch, wide));
   for (int f0 = 0; f0 < n; f0 += chunk) {
     const int m = std::min(chunk, n - f0);
-    CHK(pc_spectra(pc, m, pc->frame_ptrs.as<const void*>() + f0, type == SSG_16UC1, pitch));
-    HIPCHK(launch_pc_cross(pc->tmp.as<float2>(), pc->ref_spec.as<float2>(), pc->M, pc->N, m, s));
-    HIPCHK(launch_fft2(pc->tmp.as<float2>(), pc->buf.as<float2>(), pc->M, pc->N, m, pc->tw_m.as<float2>(),
-                       pc->tw_n.as<float2>(), true, s));
-    CHK(pc->pv.ensure(sizeof(float) * PC_PARTS_MAX * m));
-    CHK(pc->pi.ensure(sizeof(int) * PC_PARTS_MAX * m));
-    HIPCHK(launch_pc_peak(pc->buf.as<float2>(), pc->M, pc->N, pc->binning, m, pc->pv.as<float>(), pc->pi.as<int>(),
-                          pc->out.as<double>() + 3 * f0, s));
+    CHK(pc_rows(pc, f0, m, pc->frame_ptrs.as<const void*>(), type == SSG_16UC1, pitch, wide));
+    HIPCHK(launch_pc_cols(pc->plane.as<float2>(), pc->ref_spec.as<float2>(), pc->tw_n.as<float2>(), pc->M, pc->N,
+                          pc->bh, false, m, s));
+    HIPCHK(launch_pc_peak(pc->plane.as<float2>(), pc->tw_m.as<float2>(), pc->M, pc->N, pc->binning, m,
+                          pc->pv.as<float>(), pc->pi.as<int>(), pc->out.as<double>() + 3 * f0, s));
   }
   pc->prof.stop(s, SSG_PROF_FFT);
   HIPCHK(hipMemcpyAsync(out, pc->out.p, sizeof(double) * 3 * n, hipMemcpyDeviceToHost, s));
   HIPCHK(hipStreamSynchronize(s));
-  // algorithmic bytes: each frame read once (es B per pixel), plus the passes over the
-  // complex planes: load write, 2 x (row FFT r+w, transpose r+w, row FFT r+w), cross
-  // r+w + reference read, peak read -- 17 plane sweeps of 8 B per padded element
-  pc->prof.add_bytes(SSG_PROF_FFT, (double)n * ((double)es * pc->w * pc->h + 17.0 * 8.0 * per));
+  // algorithmic bytes: each frame read for its mean and for its rows (es B per pixel), and the sweeps
+  // over the plane (8 B per padded pixel): rows write half, columns read half and write all, peak reads
+  pc->prof.add_bytes(SSG_PROF_FFT, (double)n * (2.0 * es * pc->w * pc->h + 3.0 * 8.0 * per));
   pc->prof.collect();
   return SSG_OK;
 }

@@ -428,15 +428,19 @@ hipError_t launch_resize_linear(const float* src, int sw, int sh, float* dst, in
                                 hipStream_t s);
 
 // FFT phase correlation (ssg_fft.hip)
-hipError_t launch_fft2(float2* buf, float2* tmp, int M, int N, int nframes, const float2* tw_m, const float2* tw_n,
-                       bool inverse, hipStream_t s);
-constexpr int PC_PARTS_MAX = 64;  // blocks per frame of the phase-correlation reductions
-hipError_t launch_pc_load(const void* const* frames, bool u16, int pitch, int bw, int bh, int binning, float* mean,
-                          double* part, const float* wx, const float* wy, float2* out, int M, int N, int nframes,
-                          hipStream_t s);
-hipError_t launch_pc_cross(float2* spec, const float2* ref, int M, int N, int nframes, hipStream_t s);
-hipError_t launch_pc_peak(const float2* r, int M, int N, int binning, int nframes, float* pv, int* pi, double* out,
-                          hipStream_t s);
+constexpr int PC_PARTS_MAX = 64;  // blocks per frame of the phase correlation's mean
+// phase correlation (ssg_fft.hip): padded sizes M, N = 4 .. 4096
+int pc_groups(int M, int N);    // peak partials per frame
+size_t pc_plane(int M, int N);  // float2 elements per frame
+hipError_t launch_pc_mean(const void* const* frames, bool u16, int pitch, bool wide, int bw, int bh, int binning,
+                          float* mean, double* part, int nframes, hipStream_t s);
+hipError_t launch_pc_rows(const void* const* frames, bool u16, int pitch, bool wide, int bw, int bh, int binning,
+                          const float* mean, const float* wx, const float* wy, const float2* tw_m, float2* plane, int M,
+                          int N, int nframes, hipStream_t s);
+hipError_t launch_pc_cols(float2* plane, float2* ref, const float2* tw_n, int M, int N, int bh, bool store_only,
+                          int nframes, hipStream_t s);
+hipError_t launch_pc_peak(const float2* plane, const float2* tw_m, int M, int N, int binning, int nframes, float* pv,
+                          int* pi, double* out, hipStream_t s);
 
 // dense ECC flow (ssg_eccflow.hip)
 struct AreaGeom {  // one cv::resize INTER_AREA geometry, sw x sh -> dw x dh
