@@ -2456,6 +2456,16 @@ int bayer_batch(ssg_accumulation* a, int n, const ssg_image* frames, const ssg_r
   g.valid = a->valid.as<int>();
   g.nframes = n;
   g.st = a->bayer_state();
+  // staged tiles: units of 16 or 4 bytes that every frame's rows are made of, 31-bit offsets, and a cell
+  // of one R, its diagonal B and two G
+  const auto channel = [&](int q) { return (int)(a->pattern >> (2 * q) & 3u); };
+  for (int q = 0; q < 4; ++q)
+    if (channel(q) == 2 && channel(q ^ 3) == 0 && channel(q ^ 1) == 1 && channel(q ^ 2) == 1) {
+      g.pos_r = q;
+      uintptr_t bits = (uintptr_t)frames[0].step;
+      for (int f = 0; f < n; ++f) bits |= (uintptr_t)ptrs[f];
+      g.unit = (uint64_t)frames[0].step * a->h >= (1ull << 31) ? 0 : bits % 16 == 0 ? 16 : bits % 4 == 0 ? 4 : 0;
+    }
   a->prof.start(s);
   HIPCHK(launch_bayer_batch(motion_type, type == SSG_16UC1, g, s));
   a->prof.stop(s, SSG_PROF_ACCUMULATE);

@@ -111,13 +111,304 @@ __global__ void __launch_bounds__(256) k_bayer_add(BayerState st, const void* sr
 // (c_frame_registration.cc:1319-1338): remap of an all-255 mask (LINEAR,
 // CONSTANT 0) >= 255, eroded 5x5 with BORDER_CONSTANT 255.  Each thread holds
 // its pixels' accumulators in registers over all frames, in frame order.
-template <int MOTION, bool U16>
+//
+// k_bayer_staged takes the tiles whose source box fits BY_SH rows of SPR units (BayerBox) in every frame that
+// reaches them, k_bayer_batch the others: those that a map turns or stretches out of it.
+constexpr int BY_SH = 21;  // staged rows: 16, their lower taps, and what a rotation of about 2 degrees adds
+template <bool U16, int UNIT>
+struct BayerBox {
+  static constexpr int ES = U16 ? 2 : 4;
+  static constexpr int PER = UNIT / ES;                        // elements of a unit
+  static constexpr int SPR = (BY_TW + 4 + PER - 1) / PER + 1;  // units of a staged row
+  static constexpr int LOADS = (BY_SH * SPR + 255) / 256;      // units per thread
+};
+
+// the extremes of a map over a rectangle (the maps are affine: at its corners); NaN positions give a
+// rectangle that is inside nothing
+template <int MOTION>
+__device__ __forceinline__ void map_extremes(const MapCoef& mc, int rx0, int ry0, int rx1, int ry1, float& mnx,
+                                             float& mxx, float& mny, float& mxy) {
+  mnx = 1e30f, mxx = -1e30f, mny = 1e30f, mxy = -1e30f;
+  const int cx[4] = {rx0, rx1, rx0, rx1}, cy[4] = {ry0, ry0, ry1, ry1};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float sx, sy;
+    warp_xy<MOTION>(mc, cx[i], cy[i], sx, sy);
+    mnx = fminf(mnx, sx); mxx = fmaxf(mxx, sx); mny = fminf(mny, sy); mxy = fmaxf(mxy, sy);
+    if (sx != sx || sy != sy) mnx = -1e30f;
+  }
+}
+
+// the tile and its erosion halo map strictly inside the frame: no mask test
+template <int MOTION>
+__device__ __forceinline__ bool bayer_interior(const BayerState& st, const MapCoef& mc, int x0, int y0) {
+  float mnx, mxx, mny, mxy;
+  map_extremes<MOTION>(mc, max(x0 - 2, 0), max(y0 - 2, 0), min(x0 + BY_TW + 1, st.w - 1),
+                       min(y0 + BY_TH + 1, st.h - 1), mnx, mxx, mny, mxy);
+  return mnx >= 0.25f && mny >= 0.25f && mxx <= (float)st.w - 1.25f && mxy <= (float)st.h - 1.25f;
+}
+
+// What a frame is to a tile: outside (its positions all beyond the frame, or NaN: no pixel is added), staged
+// inside, staged with pixels the mask may drop, or a source box that does not fit.  The box starts at a unit
+// boundary; the corners' positions may round apart from a pixel's by less than 1/4 px.
+enum : int { BY_OUTSIDE = 0, BY_INSIDE = 1, BY_BORDER = 2, BY_UNFIT = 3 };
+template <int MOTION, bool U16, int UNIT>
+__device__ __forceinline__ int bayer_plan(const BayerState& st, const MapCoef& mc, int x0, int y0, int& bx, int& by) {
+  using Box = BayerBox<U16, UNIT>;
+  float mnx, mxx, mny, mxy;
+  map_extremes<MOTION>(mc, x0, y0, min(x0 + BY_TW - 1, st.w - 1), min(y0 + BY_TH - 1, st.h - 1), mnx, mxx, mny, mxy);
+  if (!(mnx > -1e29f) || !(mxx > -1.f) || !(mxy > -1.f) || !(mnx < (float)st.w) || !(mny < (float)st.h)) return BY_OUTSIDE;
+  if (!(mnx > -4096.f && mny > -4096.f && mxx < (float)st.w + 4096.f && mxy < (float)st.h + 4096.f)) return BY_UNFIT;
+  const int ix = (int)floorf(mnx - 0.25f);
+  bx = ix - ((ix % Box::PER) + Box::PER) % Box::PER;
+  by = (int)floorf(mny - 0.25f);
+  if ((int)floorf(mxx + 0.25f) + 1 - bx >= Box::SPR * Box::PER || (int)floorf(mxy + 0.25f) + 1 - by >= BY_SH)
+    return BY_UNFIT;
+  return bayer_interior<MOTION>(st, mc, x0, y0) ? BY_INSIDE : BY_BORDER;
+}
+
+// whether every frame of the batch fits the tile's box (the same on every lane); a translation's always do
+template <int MOTION, bool U16, int UNIT>
+__device__ __forceinline__ bool bayer_all_fit(const BayerBatchArgs& a, int x0, int y0, int lane) {
+  for (int k0 = 0; k0 < a.nframes; k0 += WAVE) {
+    const int k = k0 + lane;
+    bool ok = true;
+    if (k < a.nframes && a.valid[k]) {
+      MapCoef mc;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) mc.c[i] = a.maps[k].c[i];
+      int bx, by;
+      ok = bayer_plan<MOTION, U16, UNIT>(a.st, mc, x0, y0, bx, by) != BY_UNFIT;
+    }
+    if (!__all(ok)) return false;
+  }
+  return true;
+}
+
+// the eroded mask of a tile that is not inside the frame, into rmk: bit columns combined over x, five rows
+// of it to combine over y (barriers)
+template <int MOTION>
+__device__ __forceinline__ void bayer_mask(const BayerState& st, const MapCoef& mc, int x0, int y0,
+                                           uint8_t (*mk)[BY_TW + 4], uint8_t (*rmk)[BY_TW]) {
+  for (int i = threadIdx.x; i < (BY_TH + 4) * (BY_TW + 4); i += 256) {
+    const int ly = i / (BY_TW + 4), lx = i - ly * (BY_TW + 4);
+    const int px = x0 - 2 + lx, py = y0 - 2 + ly;
+    uint8_t v = 1;  // outside the destination: the erosion border value 255
+    if ((unsigned)px < (unsigned)st.w && (unsigned)py < (unsigned)st.h) {
+      float sx, sy;
+      warp_xy<MOTION>(mc, px, py, sx, sy);
+      v = remap_mask_u8(nullptr, 0, st.w, st.h, quant32(sx), quant32(sy)) >= 255;
+    }
+    mk[ly][lx] = v;
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < (BY_TH + 4) * BY_TW; i += 256) {
+    const int ly = i / BY_TW, lx = i - ly * BY_TW;
+    rmk[ly][lx] = mk[ly][lx] & mk[ly][lx + 1] & mk[ly][lx + 2] & mk[ly][lx + 3] & mk[ly][lx + 4];
+  }
+  __syncthreads();
+}
+
+// The staged tiles: a frame's source box goes to LDS by direct-to-LDS loads of UNIT bytes, the next frame's
+// landing while this one's taps are summed (two boxes; one barrier a frame).  The four taps of a pixel fall
+// on the four positions of the Bayer cell -- one R, one B, two G -- so each tap is read by channel, at the
+// column and row of its parity, and every update is made once, without a mask; (double)(raw * scale) * s is
+// fma(raw * s, scale, acc), the scale being a power of two.  A wave finds the boxes of 64 frames at a time,
+// a frame per lane.
+// What bounds it: vector operations, most of them the double-precision updates and their conversions.
+// 32 raw frames of 4096x3000: 1.16 ms; 2.16 ms with sixteen two-byte gathers in flight per thread and the
+// channel as a lane mask over three updates per tap (k_bayer_batch).
+// EDGE: frames whose mask may drop pixels of the tile are among them (a kernel of its own code: the
+// branches around a row's update keep its loads apart)
+template <int MOTION, bool U16, int UNIT, bool EDGE>
+__device__ __forceinline__ void bayer_tile(const BayerBatchArgs& a, int x0, int y0, int lane, int wv,
+                                           uint8_t (*box)[BayerBox<U16, UNIT>::LOADS * 256 * UNIT],
+                                           uint8_t (*mk)[BY_TW + 4], uint8_t (*rmk)[BY_TW]) {
+  using Box = BayerBox<U16, UNIT>;
+  constexpr int BP = Box::SPR * Box::PER;  // elements of a box row
+  const BayerState& st = a.st;
+  // pixels past the frame's edge repeat its last column or row; they are not stored
+  const int x = x0 + lane, xc = min(x, st.w - 1);
+  float acc[BY_RPT][3], cntr[BY_RPT][3];
+  unsigned full[BY_RPT];    // frames whose row has no zero weight: a count each for B and R, two for G
+  unsigned part[BY_RPT][3]; // counts of the other frames
+#pragma unroll
+  for (int r = 0; r < BY_RPT; ++r) {
+    const size_t o = (size_t)min(y0 + wv * BY_RPT + r, st.h - 1) * st.w + xc;
+    full[r] = 0;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      acc[r][c] = st.acc[(size_t)c * st.plane + o];
+      cntr[r][c] = st.cntr[(size_t)c * st.plane + o];
+      part[r][c] = 0;
+    }
+  }
+  const int posx = a.pos_r & 1, posy = a.pos_r >> 1;
+  const double dscale = U16 ? (double)a.scale : 1.0;
+  const uint32_t rowb = (uint32_t)a.src_pitch * Box::ES;
+  for (int k0 = 0; k0 < a.nframes; k0 += WAVE) {
+    int bx = 0, by = 0;
+    const int kl = k0 + lane;
+    int plan = BY_OUTSIDE;
+    if (kl < a.nframes && a.valid[kl]) {
+      MapCoef mc;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) mc.c[i] = a.maps[kl].c[i];
+      plan = bayer_plan<MOTION, U16, UNIT>(st, mc, x0, y0, bx, by);
+    }
+    unsigned long long left = __ballot(plan == BY_INSIDE || plan == BY_BORDER);
+    const unsigned long long border = __ballot(plan == BY_BORDER);
+    if (!left) continue;
+    auto stage = [&](int j, int buf) {  // the box of frame k0 + j
+      const int jx = __builtin_amdgcn_readlane(bx, j), jy = __builtin_amdgcn_readlane(by, j);
+      const rsrc_t rs = make_rsrc(a.frames[k0 + j], (uint32_t)st.h * rowb);
+#pragma unroll
+      for (int n = 0; n < Box::LOADS; ++n) {
+        const int i = n * 256 + wv * WAVE + lane, row = i / Box::SPR, col = i - row * Box::SPR;
+        // a unit that holds a pixel of the row lies in the row's memory (its start is a multiple of UNIT)
+        if (row < BY_SH && (unsigned)(jy + row) < (unsigned)st.h && (unsigned)(jx + col * Box::PER) < (unsigned)st.w) {
+          const uint32_t o = (uint32_t)(jy + row) * rowb + (uint32_t)(jx + col * Box::PER) * Box::ES;
+          uint8_t* d = &box[buf][(n * 256 + wv * WAVE) * UNIT];
+          if constexpr (UNIT == 16) bload_lds16(rs, d, o);
+          else bload_lds4(rs, d, o);
+        }
+      }
+    };
+    int cur = 0;
+    __syncthreads();  // the previous group's last box has been read
+    stage(__builtin_ctzll(left), 0);
+    for (; left; left &= left - 1, cur ^= 1) {
+      const int j = __builtin_ctzll(left);
+      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's part of the box has landed
+      __syncthreads();                     // every wave's has, and the other box has been read
+      if (left & (left - 1)) stage(__builtin_ctzll(left & (left - 1)), cur ^ 1);
+      const int jx = __builtin_amdgcn_readlane(bx, j), jy = __builtin_amdgcn_readlane(by, j);
+      MapCoef mc;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) mc.c[i] = a.maps[k0 + j].c[i];
+      const bool edge = EDGE && (border >> j & 1) != 0;
+      if (edge) bayer_mask<MOTION>(st, mc, x0, y0, mk, rmk);  // its barriers keep the frames' masks apart
+      auto raw = [&](int o) {
+        if constexpr (U16) return (double)((const uint16_t*)box[cur])[o];
+        else return (double)((const float*)box[cur])[o];
+      };
+      int sx = 0, cr = 0;
+      double wxr = 0, wxb = 0;
+      bool xnz = true;
+      auto columns = [&](float px) {  // R's column is that of its parity, B's the other one
+        sx = (int)px;
+        const float ax = (float)(sx + 1) - px, bxf = px - (float)sx;
+        cr = (sx ^ posx) & 1;
+        wxr = (double)(cr ? bxf : ax);
+        wxb = (double)(cr ? ax : bxf);
+        xnz = bxf != 0.f;
+      };
+      if constexpr (MOTION == MOTION_TRANSLATION) columns((float)xc + mc.c[0]);
+#pragma unroll
+      for (int r = 0; r < BY_RPT; ++r) {
+        float px, py;
+        warp_xy<MOTION>(mc, xc, min(y0 + wv * BY_RPT + r, st.h - 1), px, py);
+        if constexpr (MOTION != MOTION_TRANSLATION) columns(px);
+        const int sy = (int)py;
+        const float ay = (float)(sy + 1) - py, byf = py - (float)sy;
+        const bool below = ((sy ^ posy) & 1) != 0;  // R lies in row sy + 1
+        const double wyr = (double)(below ? byf : ay), wyb = (double)(below ? ay : byf);
+        if (edge) {
+          const int ly = wv * BY_RPT + r;
+          if (!(rmk[ly][lane] & rmk[ly + 1][lane] & rmk[ly + 2][lane] & rmk[ly + 3][lane] & rmk[ly + 4][lane])) continue;
+          if (!(sx >= 0 && sx < st.w - 1 && sy >= 0 && sy < st.h - 1)) continue;
+        }
+        const int o0 = (sy - jy) * BP + sx - jx, cb = 1 - cr;
+        const double sr = wxr * wyr, sb = wxb * wyb, p = wxb * wyr, q = wxr * wyb;
+        const double s1 = below ? q : p, s2 = below ? p : q;  // the G taps of rows sy and sy + 1, in that order
+        const double vr = raw(o0 + cr + (below ? BP : 0)), vb = raw(o0 + cb + (below ? 0 : BP));
+        const double v1 = raw(o0 + (below ? cr : cb)), v2 = raw(o0 + BP + (below ? cb : cr));
+        acc[r][2] = (float)fma(vr * sr, dscale, (double)acc[r][2]);
+        acc[r][0] = (float)fma(vb * sb, dscale, (double)acc[r][0]);
+        acc[r][1] = (float)fma(v1 * s1, dscale, (double)acc[r][1]);
+        acc[r][1] = (float)fma(v2 * s2, dscale, (double)acc[r][1]);
+        cntr[r][2] = (float)((double)cntr[r][2] + sr);
+        cntr[r][0] = (float)((double)cntr[r][0] + sb);
+        cntr[r][1] = (float)((double)cntr[r][1] + s1);
+        cntr[r][1] = (float)((double)cntr[r][1] + s2);
+        // ax, ay > 0: a weight is zero only where a lower tap's factor is
+        if (!edge && __all(xnz && byf != 0.f)) {
+          full[r] += 1;
+        } else {
+          part[r][2] += sr != 0.0;
+          part[r][0] += sb != 0.0;
+          part[r][1] += (s1 != 0.0) + (s2 != 0.0);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < BY_RPT; ++r) {
+    const int y = y0 + wv * BY_RPT + r;
+    if (x >= st.w || y >= st.h) continue;
+    const size_t o = (size_t)y * st.w + x;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      st.acc[(size_t)c * st.plane + o] = acc[r][c];
+      st.cntr[(size_t)c * st.plane + o] = cntr[r][c];
+      st.cnt[(size_t)c * st.plane + o] += part[r][c] + (c == 1 ? 2 * full[r] : full[r]);
+    }
+  }
+}
+
+template <int MOTION, bool U16, int UNIT>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_bayer_staged(BayerBatchArgs a) {
+  // a wave's loads write WAVE consecutive units from a uniform base
+  __shared__ __align__(16) uint8_t box[2][BayerBox<U16, UNIT>::LOADS * 256 * UNIT];
+  __shared__ uint8_t mk[BY_TH + 4][BY_TW + 4];
+  __shared__ uint8_t rmk[BY_TH + 4][BY_TW];
+  const int lane = threadIdx.x & (WAVE - 1), wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x / WAVE);
+  // the outermost ring of tiles first: the masks make them three times as long as the others, and the last
+  // ones would be the launch's tail; then the inner tiles row by row
+  const int X = (a.st.w + BY_TW - 1) / BY_TW, Y = (a.st.h + BY_TH - 1) / BY_TH, id = blockIdx.x;
+  int tx, ty;
+  if (X < 3 || Y < 3) {
+    tx = id % X, ty = id / X;
+  } else if (id < 2 * X) {
+    tx = id % X, ty = id < X ? 0 : Y - 1;
+  } else if (id < 2 * X + 2 * (Y - 2)) {
+    const int i = id - 2 * X;
+    tx = i & 1 ? X - 1 : 0, ty = 1 + (i >> 1);
+  } else {
+    const int i = id - 2 * X - 2 * (Y - 2);
+    tx = 1 + i % (X - 2), ty = 1 + i / (X - 2);
+  }
+  const int x0 = tx * BY_TW, y0 = ty * BY_TH;
+  bool fit = true, inside = true;
+  for (int k0 = 0; k0 < a.nframes; k0 += WAVE) {
+    const int k = k0 + lane;
+    int plan = BY_INSIDE;
+    if (k < a.nframes && a.valid[k]) {
+      MapCoef mc;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) mc.c[i] = a.maps[k].c[i];
+      int bx, by;
+      plan = bayer_plan<MOTION, U16, UNIT>(a.st, mc, x0, y0, bx, by);
+    }
+    fit = fit && __all(plan != BY_UNFIT);
+    inside = inside && __all(plan == BY_INSIDE || plan == BY_OUTSIDE);
+  }
+  if (!fit) return;
+  if (inside) bayer_tile<MOTION, U16, UNIT, false>(a, x0, y0, lane, wv, box, mk, rmk);
+  else bayer_tile<MOTION, U16, UNIT, true>(a, x0, y0, lane, wv, box, mk, rmk);
+}
+
+// The other tiles (UNIT as of the k_bayer_staged launched before it; 0: all tiles).
+template <int MOTION, bool U16, int UNIT>
 __global__ void __launch_bounds__(256) k_bayer_batch(BayerBatchArgs a) {
   __shared__ uint8_t mk[BY_TH + 4][BY_TW + 4];
   __shared__ uint8_t rmk[BY_TH + 4][BY_TW];
   const BayerState& st = a.st;
   const int tid = threadIdx.x, lane = tid & (WAVE - 1), wv = tid / WAVE;
   const int x0 = blockIdx.x * BY_TW, y0 = blockIdx.y * BY_TH;
+  if constexpr (UNIT > 0) {
+    if (bayer_all_fit<MOTION, U16, UNIT>(a, x0, y0, lane)) return;
+  }
   const int x = x0 + lane;
   float acc[BY_RPT][3], cntr[BY_RPT][3];
   unsigned cnt[BY_RPT][3];
@@ -139,39 +430,9 @@ __global__ void __launch_bounds__(256) k_bayer_batch(BayerBatchArgs a) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) mc.c[i] = a.maps[k].c[i];
     const void* src = a.frames[k];
-    // uniform test: the tile and its erosion halo map strictly inside the frame
-    const int ex0 = max(x0 - 2, 0), ey0 = max(y0 - 2, 0);
-    const int ex1 = min(x0 + BY_TW + 1, st.w - 1), ey1 = min(y0 + BY_TH + 1, st.h - 1);
-    float mnx = 1e30f, mxx = -1e30f, mny = 1e30f, mxy = -1e30f;
-    {
-      const int cx[4] = {ex0, ex1, ex0, ex1}, cy[4] = {ey0, ey0, ey1, ey1};
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float sx, sy;
-        warp_xy<MOTION>(mc, cx[i], cy[i], sx, sy);
-        mnx = fminf(mnx, sx); mxx = fmaxf(mxx, sx); mny = fminf(mny, sy); mxy = fmaxf(mxy, sy);
-        if (sx != sx || sy != sy) mnx = -1e30f;  // NaN positions take the bordered path
-      }
-    }
-    const bool interior = mnx >= 0.25f && mny >= 0.25f && mxx <= (float)st.w - 1.25f && mxy <= (float)st.h - 1.25f;
+    const bool interior = bayer_interior<MOTION>(st, mc, x0, y0);
     if (!interior) {
-      for (int i = tid; i < (BY_TH + 4) * (BY_TW + 4); i += 256) {
-        const int ly = i / (BY_TW + 4), lx = i - ly * (BY_TW + 4);
-        const int px = x0 - 2 + lx, py = y0 - 2 + ly;
-        uint8_t v = 1;  // outside the destination: the erosion border value 255
-        if ((unsigned)px < (unsigned)st.w && (unsigned)py < (unsigned)st.h) {
-          float sx, sy;
-          warp_xy<MOTION>(mc, px, py, sx, sy);
-          v = remap_mask_u8(nullptr, 0, st.w, st.h, quant32(sx), quant32(sy)) >= 255;
-        }
-        mk[ly][lx] = v;
-      }
-      __syncthreads();
-      for (int i = tid; i < (BY_TH + 4) * BY_TW; i += 256) {
-        const int ly = i / BY_TW, lx = i - ly * BY_TW;
-        rmk[ly][lx] = mk[ly][lx] & mk[ly][lx + 1] & mk[ly][lx + 2] & mk[ly][lx + 3] & mk[ly][lx + 4];
-      }
-      __syncthreads();
+      bayer_mask<MOTION>(st, mc, x0, y0, mk, rmk);
     }
 #pragma unroll
     for (int r = 0; r < BY_RPT; ++r) {
@@ -265,10 +526,20 @@ hipError_t launch_bayer_add(const BayerState& st, const void* src, int src_pitch
 
 hipError_t launch_bayer_batch(int motion, bool u16, const BayerBatchArgs& a, hipStream_t s) {
   dim3 grid((a.st.w + BY_TW - 1) / BY_TW, (a.st.h + BY_TH - 1) / BY_TH);
-#define SSG_BB(M)                                                                     \
-  do {                                                                                \
-    if (u16) hipLaunchKernelGGL((k_bayer_batch<M, true>), grid, dim3(256), 0, s, a);  \
-    else hipLaunchKernelGGL((k_bayer_batch<M, false>), grid, dim3(256), 0, s, a);     \
+#define SSG_BB2(M, U, UNIT)                                                               \
+  do {                                                                                    \
+    if (UNIT) hipLaunchKernelGGL((k_bayer_staged<M, U, UNIT ? UNIT : 4>), dim3(grid.x * grid.y), dim3(256), 0, s, a); \
+    if (!UNIT || M != MOTION_TRANSLATION)                                                 \
+      hipLaunchKernelGGL((k_bayer_batch<M, U, UNIT>), grid, dim3(256), 0, s, a);          \
+  } while (0)
+#define SSG_BB(M)                                 \
+  do {                                            \
+    if (a.unit == 16 && u16) SSG_BB2(M, true, 16);    \
+    else if (a.unit == 16) SSG_BB2(M, false, 16);     \
+    else if (a.unit == 4 && u16) SSG_BB2(M, true, 4); \
+    else if (a.unit == 4) SSG_BB2(M, false, 4);       \
+    else if (u16) SSG_BB2(M, true, 0);                \
+    else SSG_BB2(M, false, 0);                        \
   } while (0)
   switch (motion) {
     case MOTION_TRANSLATION: SSG_BB(MOTION_TRANSLATION); break;
@@ -278,6 +549,7 @@ hipError_t launch_bayer_batch(int motion, bool u16, const BayerBatchArgs& a, hip
     default: return hipErrorInvalidValue;
   }
 #undef SSG_BB
+#undef SSG_BB2
   return hipGetLastError();
 }
 

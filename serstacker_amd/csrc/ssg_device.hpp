@@ -33,6 +33,14 @@ __device__ __forceinline__ float bload_f32(rsrc_t r, uint32_t voff, uint32_t sof
   return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
 }
 
+// direct-to-LDS loads of 16 or 4 bytes per lane: lane l's go to lds + l * their size, lds being uniform
+__device__ __forceinline__ void bload_lds16(rsrc_t r, void* lds, uint32_t voff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, voff, 0, 0, 0);
+}
+__device__ __forceinline__ void bload_lds4(rsrc_t r, void* lds, uint32_t voff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 4, voff, 0, 0, 0);
+}
+
 // cv::borderInterpolate; -1 for CONSTANT/TRANSPARENT
 __device__ __forceinline__ int border_interp(int p, int len, int border) {
   if ((unsigned)p < (unsigned)len) return p;

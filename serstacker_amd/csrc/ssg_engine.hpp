@@ -286,6 +286,8 @@ struct BayerBatchArgs {
   const MapCoef* maps;
   const int* valid;
   int nframes;
+  int unit;                   // 16 or 4: every row of every frame starts at a multiple of so many bytes; 0: none
+  int pos_r;                  // position of R in the Bayer cell ((y & 1) << 1 | (x & 1)), B diagonal to it
   BayerState st;
 };
 
