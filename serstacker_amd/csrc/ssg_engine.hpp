@@ -424,6 +424,14 @@ hipError_t launch_morph_grad(const float* m, int w, int h, int r, float* g, hipS
 hipError_t launch_int_to_f32(const void* src, int pitch, int w, int h, bool u16, float* dst, hipStream_t s);
 hipError_t launch_round_half_up(float* v, size_t n, hipStream_t s);
 int lvm_sum_blocks(size_t n);
+// quality of n 8/16-bit frames of aw x ah pixels (bayer: cells of the raw frame): their pyrDown in whole numbers
+// stored dense (out), or its gradient's sums of G and G^4 (part: quality_tiles pairs a frame; sums: a pair).
+// The frames by a table of pointers, or (fstride != 0) planes fstride bytes apart from `frames` on; wide: two
+// pixels' samples lie at an address that is a multiple of their bytes, in every row of every frame
+int quality_max_radius();
+int quality_tiles(int dw, int dh, int r);
+hipError_t launch_quality(const void* const* frames, long long fstride, bool u16, bool bayer, int pitch, bool wide, int aw,
+                          int ah, int r, int n, uint16_t* out, double* part, double* sums, hipStream_t s);
 hipError_t launch_lvm_sums(const float* g, size_t n, double* partial, hipStream_t s);
 hipError_t launch_lvm_map(const float* g, size_t n, float map_scale, float add, float* m, hipStream_t s);
 hipError_t launch_resize_linear(const float* src, int sw, int sh, float* dst, int dst_pitch, int dw, int dh,
