@@ -131,19 +131,22 @@ __device__ __forceinline__ float hup(const float* S, int sw, int xo) {
   return fmaf(S[x * ST], 6.f, S[(x - 1) * ST] + S[(x + 1) * ST]);
 }
 
-// sum of p[t * elem_stride] for t = t0, t0 + stride, ... < n, added in that order, with eight
-// loads in flight ahead of the additions (the same sum as the plain loop, bit for bit)
+// sum of p[t * elem_stride] for t = t0, t0 + stride, ... < n, added in that order, with a batch of
+// loads in flight ahead of the additions: 32 while more than eight are left, else eight (the same
+// sum as the plain loop, bit for bit; the loads past the end repeat the last value, not added)
+template <int N>
+__device__ __forceinline__ void ordered_batch(const double* p, int t, int n, int stride, int elem_stride, double& s) {
+  double v[N];
+#pragma unroll
+  for (int u = 0; u < N; ++u) v[u] = p[(size_t)min(t + u * stride, n - 1) * elem_stride];
+#pragma unroll
+  for (int u = 0; u < N; ++u) s = t + u * stride < n ? s + v[u] : s;
+}
 __device__ __forceinline__ double ordered_strided_sum(const double* p, int t0, int n, int stride, int elem_stride) {
   double s = 0;
   int t = t0;
-  for (; t + 7 * stride < n; t += 8 * stride) {
-    double v[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = p[(size_t)(t + u * stride) * elem_stride];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) s += v[u];
-  }
-  for (; t < n; t += stride) s += p[(size_t)t * elem_stride];
+  for (; t + 8 * stride < n; t += 32 * stride) ordered_batch<32>(p, t, n, stride, elem_stride, s);
+  if (t < n) ordered_batch<8>(p, t, n, stride, elem_stride, s);
   return s;
 }
 

@@ -116,20 +116,12 @@ __device__ double expand_moment(int k, const float* loc, double X0, double Y0) {
   return loc[k];
 }
 
-// Solve of one ECC iteration (ecc2.cc:1320-1362) from the frame's moments.
-// Runs on one thread; every matrix lives in the LDS scratch sm (the moments G
-// occupy sm[0..63]) so the hot path of the kernel keeps its register budget.
+// Solve of one ECC iteration (ecc2.cc:1320-1362) from the frame's moments G (LDS).
+// A chain of dependent FP64 operations on one thread: every matrix is in registers and every
+// loop unrolled, so that the independent divisions of a column overlap and no step waits for
+// LDS.  The lane that writes reports into R.
 template <int MOTION, bool FULL>
-__device__ void ecc_solve(double* sm, FrameXf& X, FrameRes& R, const EccPassArgs& a) {
-  const double* G = sm;
-  double* Ha = sm + 64;   // 6x6
-  double* H = sm + 100;   // NP x NP
-  double* L = sm + 136;   // NP x NP
-  double* T = sm + 172;   // NP x 6
-  double* M = sm + 208;   // NP x 6
-  double* ea = sm + 244;  // 6
-  double* e = sm + 250;   // NP
-  double* z = sm + 256;   // NP
+__device__ __forceinline__ void ecc_solve(const double* G, FrameXf& X, FrameRes& R, const EccPassArgs& a, bool write) {
   // ---- masked statistics (cv::meanStdDev, population stdev)
   double n, sf, sff, sg, sgg;
   if (FULL) {
@@ -146,6 +138,7 @@ __device__ void ecc_solve(double* sm, FrameXf& X, FrameRes& R, const EccPassArgs
 
   constexpr int NP = MOTION == MOTION_TRANSLATION ? 2
                      : (MOTION == MOTION_EUCLIDEAN ? 3 : (MOTION == MOTION_SCALED_EUCLIDEAN ? 4 : 6));
+  double H[NP * NP], e[NP], z[NP];
   if (!FULL) {
     // J = [gx, gy]
     H[0] = G[0]; H[1] = G[1]; H[2] = G[1]; H[3] = G[2];
@@ -160,9 +153,13 @@ __device__ void ecc_solve(double* sm, FrameXf& X, FrameRes& R, const EccPassArgs
                                              Cc[3], Cc[4], Cc[1],
                                                     Cc[5], Cc[2],
                                                            Cc[0]};
-    for (int i = 0, q = 0; i < 6; ++i)
-      for (int j = i; j < 6; ++j, ++q) Ha[i * 6 + j] = Ha[j * 6 + i] = up[q];
+    double Ha[36], ea[6];
+#pragma unroll
+    for (int i = 0; i < 6; ++i)
+#pragma unroll
+      for (int j = i; j < 6; ++j) Ha[i * 6 + j] = Ha[j * 6 + i] = up[i * 6 - i * (i - 1) / 2 + j - i];
     const double *P = G + 18, *Q = G + 21, *Rr = G + 24, *S = G + 27, *GX = G + 30, *GY = G + 33;
+#pragma unroll
     for (int i = 0; i < 6; ++i) {
       const int k = (i % 3 == 0) ? 1 : ((i % 3 == 1) ? 2 : 0);  // X, Y, 1
       const double bg = i < 3 ? P[k] : Q[k];
@@ -171,10 +168,14 @@ __device__ void ecc_solve(double* sm, FrameXf& X, FrameRes& R, const EccPassArgs
       ea[i] = bg - ratio * bf - kc * b1;
     }
     if (MOTION == MOTION_AFFINE) {
-      for (int i = 0; i < 36; ++i) H[i] = Ha[i];
-      for (int i = 0; i < 6; ++i) e[i] = ea[i];
+#pragma unroll
+      for (int i = 0; i < NP * NP; ++i) H[i] = Ha[i];
+#pragma unroll
+      for (int i = 0; i < NP; ++i) e[i] = ea[i];
     } else {
       // J = M J_aff (c_image_transform.cc:587-668 rewritten on the affine basis)
+      double M[NP * 6], T[NP * 6];
+#pragma unroll
       for (int i = 0; i < NP * 6; ++i) M[i] = 0;
       M[0 * 6 + 2] = 1;
       M[1 * 6 + 5] = 1;
@@ -187,18 +188,25 @@ __device__ void ecc_solve(double* sm, FrameXf& X, FrameRes& R, const EccPassArgs
           M[3 * 6 + 3] = sa; M[3 * 6 + 4] = ca;  M[3 * 6 + 5] = -(sa * Cx + ca * Cy);
         }
       }
+#pragma unroll
       for (int i = 0; i < NP; ++i)
+#pragma unroll
         for (int j = 0; j < 6; ++j) {
           double t = 0;
+#pragma unroll
           for (int k = 0; k < 6; ++k) t += M[i * 6 + k] * Ha[k * 6 + j];
           T[i * 6 + j] = t;
         }
+#pragma unroll
       for (int i = 0; i < NP; ++i) {
         double t = 0;
+#pragma unroll
         for (int k = 0; k < 6; ++k) t += M[i * 6 + k] * ea[k];
         e[i] = t;
+#pragma unroll
         for (int j = 0; j < NP; ++j) {
           double u = 0;
+#pragma unroll
           for (int k = 0; k < 6; ++k) u += T[i * 6 + k] * M[j * 6 + k];
           H[i * NP + j] = u;
         }
@@ -232,45 +240,58 @@ __device__ void ecc_solve(double* sm, FrameXf& X, FrameRes& R, const EccPassArgs
       inv[7] = (H[1] * H[6] - H[0] * H[7]) * r;
       inv[8] = (H[0] * H[4] - H[1] * H[3]) * r;
     }
+#pragma unroll
     for (int i = 0; i < NP; ++i) {
       double t = 0;
+#pragma unroll
       for (int j = 0; j < NP; ++j) t += inv[i * NP + j] * e[j];
       z[i] = t;
     }
   } else {
-    for (int i = 0; i < NP && !failed; ++i) {
+    // a failed pivot leaves the rest of the values unused
+    double L[NP * NP];
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+#pragma unroll
       for (int j = 0; j < i; ++j) {
         double s = H[i * NP + j];
+#pragma unroll
         for (int k = 0; k < j; ++k) s -= L[i * NP + k] * L[j * NP + k];
         L[i * NP + j] = s / L[j * NP + j];
       }
       double s = H[i * NP + i];
+#pragma unroll
       for (int k = 0; k < i; ++k) s -= L[i * NP + k] * L[i * NP + k];
-      if (s < (double)FLT_EPSILON) failed = true;
-      else L[i * NP + i] = sqrt(s);
+      failed = failed || s < (double)FLT_EPSILON;
+      L[i * NP + i] = sqrt(s);
     }
-    if (!failed) {
-      for (int i = 0; i < NP; ++i) {
-        double s = e[i];
-        for (int j = 0; j < i; ++j) s -= L[i * NP + j] * z[j];
-        z[i] = s / L[i * NP + i];
-      }
-      for (int i = NP - 1; i >= 0; --i) {
-        double s = z[i];
-        for (int j = i + 1; j < NP; ++j) s -= L[j * NP + i] * z[j];
-        z[i] = s / L[i * NP + i];
-      }
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      double s = e[i];
+#pragma unroll
+      for (int j = 0; j < i; ++j) s -= L[i * NP + j] * z[j];
+      z[i] = s / L[i * NP + i];
+    }
+#pragma unroll
+    for (int i = NP - 1; i >= 0; --i) {
+      double s = z[i];
+#pragma unroll
+      for (int j = i + 1; j < NP; ++j) s -= L[j * NP + i] * z[j];
+      z[i] = s / L[i * NP + i];
     }
   }
   X.iters += 1;
   const int k = X.iters;
   if (failed) {
-    R.level_iters[a.pass][a.level] = k;
-    R.level_failed[a.pass][a.level] = 1;
+    if (write) {
+      R.level_iters[a.pass][a.level] = k;
+      R.level_failed[a.pass][a.level] = 1;
+    }
     X.flags &= ~XF_ACTIVE;
     return;
   }
   float dp[6] = {0, 0, 0, 0, 0, 0};
+#pragma unroll
   for (int i = 0; i < NP; ++i) {
     dp[i] = (float)(-a.update_step_scale * z[i]);
     X.p[i] = X.p[i] + dp[i];
@@ -279,13 +300,13 @@ __device__ void ecc_solve(double* sm, FrameXf& X, FrameRes& R, const EccPassArgs
   X.cg = (float)((double)X.cg + mg);
   const float eps = xf_eps(MOTION, dp, a.w, a.h);
   X.eps = eps;
-  R.eps = eps;
+  if (write) R.eps = eps;
   if (eps < a.max_eps) {
-    R.level_iters[a.pass][a.level] = k;
+    if (write) R.level_iters[a.pass][a.level] = k;
     X.flags &= ~XF_ACTIVE;
   } else if (k >= a.max_iterations) {
     // while (_num_iterations++ < _max_iterations): exhaustion leaves max + 1
-    R.level_iters[a.pass][a.level] = k + 1;
+    if (write) R.level_iters[a.pass][a.level] = k + 1;
     X.flags &= ~XF_ACTIVE;
   }
 }
@@ -334,75 +355,113 @@ __device__ __forceinline__ bool translation_key(float t, int n, int& q) {
 // order (deterministic), solves, and appends the frame to the next active
 // list while it keeps iterating.  A translation goes on solving here while its
 // new position is one whose moments it has kept (EccMemo): those iterations
-// cost no pass and give the pass's own result, bit for bit.  192 frames of
-// 1080p, four levels: translation passes 17.1 -> 5.6 ms, their solves 1.3 -> 1.8 ms.  Runs after k_ecc_pass, so the kernel
+// cost no pass and give the pass's own result, bit for bit (192 frames of 1080p, four
+// levels: translation passes 17.1 -> 5.6 ms).  The chain of such iterations runs in one wave with
+// the kept moments in LDS and their keys in its lanes, every lane doing the same solve, so
+// that an iteration waits for neither a barrier nor memory.  The launch is latency alone:
+// with the matrices in LDS, eight loads in flight and a barrier per kept iteration it took 12.2 us
+// (affine) and 9.1 us (translation) on average over 192 frames of 1080p and 25 us (translation) over
+// 640x480 frames; now 7.8, 5.8 and 13.7 us.  Runs after k_ecc_pass, so the kernel
 // boundary makes every tile's partial visible without device-scope fences.
-template <int MOTION, bool FULL>
+template <int MOTION>
 __global__ void __launch_bounds__(256) k_ecc_solve(EccPassArgs a) {
+  constexpr bool FULL = MOTION != MOTION_TRANSLATION;
   constexpr int NM = FULL ? NMOM_FULL : NMOM_TRANS;
   __shared__ double dred[ECC_WAVES][64];
-  __shared__ double s_solve[272];
+  __shared__ double G[FULL ? 1 : ECC_MEMO + 1][NM];  // the kept moments, then a position that is not kept
   const int f = blockIdx.x;
   if (!(a.xf[f].flags & XF_ACTIVE)) return;
-  const int tid = threadIdx.x, lane = tid & (WAVE - 1), wv = tid / WAVE;
+  FrameXf X;
   {
-    const int k = lane, j = wv;
-    double s = 0;
-    if (k < NM) {
-      const double* base = reinterpret_cast<const double*>(a.partials) + (size_t)f * a.ntiles * NM;
-      s = ordered_strided_sum(base + k, j, a.ntiles, ECC_WAVES, NM);
+    // field by field: a copy of the whole would live in scratch, which costs the launch 5 us
+    const FrameXf& from = a.xf[f];
+#pragma unroll
+    for (int i = 0; i < 6; ++i) X.p[i] = from.p[i];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) X.mc.c[i] = from.mc.c[i];
+    X.C[0] = from.C[0];
+    X.C[1] = from.C[1];
+    X.cg = from.cg;
+    X.iters = from.iters;
+    X.flags = from.flags;
+    X.eps = from.eps;
+  }
+  const int tid = threadIdx.x, lane = tid & (WAVE - 1), wv = __builtin_amdgcn_readfirstlane(tid / WAVE);
+  int count = 0, kx = 0, ky = 0;
+  float kc = 0.f;
+  if constexpr (!FULL) {
+    const EccMemo& M = a.memo[f];
+    count = M.count;
+    const int n = min(count, ECC_MEMO);
+    for (int i = tid; i < n * NM; i += 256) G[0][i] = M.G[0][i];
+    if (tid < n) {
+      kx = M.qx[tid];
+      ky = M.qy[tid];
+      kc = M.cg[tid];
     }
-    dred[j][k] = s;
+  }
+  {
+    double s = 0;
+    if (lane < NM) {
+      const double* base = reinterpret_cast<const double*>(a.partials) + (size_t)f * a.ntiles * NM;
+      s = ordered_strided_sum(base + lane, wv, a.ntiles, ECC_WAVES, NM);
+    }
+    dred[wv][lane] = s;
   }
   __syncthreads();
-  if (tid < NM) s_solve[tid] = ((dred[0][tid] + dred[1][tid]) + dred[2][tid]) + dred[3][tid];
-  if constexpr (!FULL) {
-    __shared__ int s_hit, s_go, s_q[4];
-    EccMemo& M = a.memo[f];
-    FrameXf X = a.xf[f];  // thread 0's copy goes through the iterations and is written back
+  if (wv != 0) return;
+  const double sum = ((dred[0][lane] + dred[1][lane]) + dred[2][lane]) + dred[3][lane];
+  int at = 0;
+  if constexpr (FULL) {
+    if (lane < NM) G[0][lane] = sum;
+  } else {
     int qx, qy;
     const bool keep = translation_key(X.p[0], a.w, qx) && translation_key(X.p[1], a.h, qy);
-    const int at = M.count % ECC_MEMO;
-    __syncthreads();
+    at = keep ? count % ECC_MEMO : ECC_MEMO;
+    if (lane < NM) G[at][lane] = sum;
     if (keep) {
-      if (tid < NM) M.G[at][tid] = s_solve[tid];
-      if (tid == 0) {
-        M.qx[at] = qx;
-        M.qy[at] = qy;
-        M.cg[at] = X.cg;
-        M.count += 1;
+      EccMemo& M = a.memo[f];
+      if (lane < NM) M.G[at][lane] = sum;
+      if (lane == at) {
+        M.qx[at] = kx = qx;
+        M.qy[at] = ky = qy;
+        M.cg[at] = kc = X.cg;
+        M.count = count + 1;
       }
+      count += 1;
     }
+  }
+  // the wave's LDS stores before its loads of other lanes' values
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+  if constexpr (FULL) {
+    ecc_solve<MOTION, FULL>(G[0], X, a.res[f], a, lane == 0);
+  } else {
     // ecc_solve ends the loop at the latest when the iteration budget is spent
     for (;;) {
-      if (tid == 0) {
-        ecc_solve<MOTION, FULL>(s_solve, X, a.res[f], a);
-        s_hit = -1;
-        s_go = (X.flags & XF_ACTIVE) && translation_key(X.p[0], a.w, qx) && translation_key(X.p[1], a.h, qy);
-        s_q[0] = qx;
-        s_q[1] = qy;
-        s_q[2] = __float_as_int(X.cg);
-        s_q[3] = min(M.count, ECC_MEMO);
-      }
-      __syncthreads();
-      if (!s_go) break;
-      if (tid < s_q[3] && M.qx[tid] == s_q[0] && M.qy[tid] == s_q[1] && __float_as_int(M.cg[tid]) == s_q[2]) s_hit = tid;
-      __syncthreads();
-      const int hit = s_hit;
-      if (hit < 0) break;
-      if (tid < NM) s_solve[tid] = M.G[hit][tid];
-      __syncthreads();  // the moments are in place; s_hit and s_go have been read
+      ecc_solve<MOTION, FULL>(G[at], X, a.res[f], a, lane == 0);
+      int qx, qy;
+      if (!(X.flags & XF_ACTIVE) || !translation_key(X.p[0], a.w, qx) || !translation_key(X.p[1], a.h, qy)) break;
+      const unsigned long long hit = __ballot(lane < min(count, ECC_MEMO) && kx == qx && ky == qy &&
+                                              __float_as_int(kc) == __float_as_int(X.cg));
+      if (hit == 0) break;
+      at = __ffsll(hit) - 1;
     }
-    if (tid == 0) a.xf[f] = X;
-  } else {
-    __syncthreads();
   }
-  if (tid == 0) {
-    if constexpr (FULL) ecc_solve<MOTION, FULL>(s_solve, a.xf[f], a.res[f], a);
-    if (a.xf[f].flags & XF_ACTIVE) {
+  if (lane == 0) {
+    FrameXf& to_xf = a.xf[f];
+#pragma unroll
+    for (int i = 0; i < 6; ++i) to_xf.p[i] = X.p[i];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) to_xf.mc.c[i] = X.mc.c[i];
+    to_xf.cg = X.cg;
+    to_xf.iters = X.iters;
+    to_xf.flags = X.flags;
+    to_xf.eps = X.eps;
+    if (X.flags & XF_ACTIVE) {
       // the list order does not affect any frame's result
-      const int at = atomicAdd(a.active_count_out, 1);
-      a.active_out[at] = f;
+      const int to = atomicAdd(a.active_count_out, 1);
+      a.active_out[to] = f;
     }
   }
 }
@@ -457,18 +516,17 @@ static hipError_t launch_pass_m(const EccPassArgs& a, bool full, int grid, hipSt
 }
 
 template <int MOTION>
-static hipError_t launch_solve_m(const EccPassArgs& a, bool full, hipStream_t s) {
-  if (full) hipLaunchKernelGGL((k_ecc_solve<MOTION, true>), dim3(a.nframes), dim3(256), 0, s, a);
-  else hipLaunchKernelGGL((k_ecc_solve<MOTION, false>), dim3(a.nframes), dim3(256), 0, s, a);
+static hipError_t launch_solve_m(const EccPassArgs& a, hipStream_t s) {
+  hipLaunchKernelGGL((k_ecc_solve<MOTION>), dim3(a.nframes), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 
 hipError_t launch_ecc_solve(int motion, const EccPassArgs& a, hipStream_t s) {
   switch (motion) {
-    case MOTION_TRANSLATION: return launch_solve_m<MOTION_TRANSLATION>(a, false, s);
-    case MOTION_EUCLIDEAN: return launch_solve_m<MOTION_EUCLIDEAN>(a, true, s);
-    case MOTION_SCALED_EUCLIDEAN: return launch_solve_m<MOTION_SCALED_EUCLIDEAN>(a, true, s);
-    case MOTION_AFFINE: return launch_solve_m<MOTION_AFFINE>(a, true, s);
+    case MOTION_TRANSLATION: return launch_solve_m<MOTION_TRANSLATION>(a, s);
+    case MOTION_EUCLIDEAN: return launch_solve_m<MOTION_EUCLIDEAN>(a, s);
+    case MOTION_SCALED_EUCLIDEAN: return launch_solve_m<MOTION_SCALED_EUCLIDEAN>(a, s);
+    case MOTION_AFFINE: return launch_solve_m<MOTION_AFFINE>(a, s);
   }
   return hipErrorInvalidValue;
 }
