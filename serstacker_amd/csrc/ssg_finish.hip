@@ -180,58 +180,84 @@ __device__ __forceinline__ float apr_rule(float fm, const float* fb, const doubl
   return m;
 }
 
+// The mask counts of the kernels below: one addition per block to the one counter, from the waves'
+// ballots.  An addition per wave kept the kernel at the rate of that one address (11 ns each: 812 us for the
+// 2880 x 1620 level, whose bytes take 20 us; now 36 us; the halvings that follow 296 -> 55 us).  Hence blocks of 64 columns by 4 x rows rows,
+// rows chosen by apr_rows so that the large levels still give four blocks per CU.
+__device__ __forceinline__ void apr_count(unsigned mine, unsigned* nz) {
+  __shared__ unsigned part[4];
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = mine;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const unsigned t = part[0] + part[1] + part[2] + part[3];
+    if (t) atomicAdd(nz, t);
+  }
+}
+
 // level 0: src.copyTo(img, mask), msk = mask * (float)(1 / 255.) (:114-115); counts the mask's
 // non-zero pixels
 template <int CN>
 __global__ void __launch_bounds__(256) k_apr_init(const float* src, int spitch, const uint8_t* mask, int mpitch, int w,
-                                                   int h, float* img, float* msk, unsigned* nz) {
-  const int x = blockIdx.x * 64 + (threadIdx.x & 63), y = blockIdx.y * 4 + (threadIdx.x >> 6);
-  bool valid = false;
-  if (x < w && y < h) {
-    const uint8_t m = mask[(size_t)y * mpitch + x];
-    valid = m != 0;
-    const float* sp = src + (size_t)y * spitch + (size_t)x * CN;
-    float* dp = img + ((size_t)y * w + x) * CN;
-    for (int c = 0; c < CN; ++c) dp[c] = valid ? sp[c] : 0.f;
-    msk[(size_t)y * w + x] = (float)m * (float)(1.0 / 255.0);
+                                                   int h, float* img, float* msk, unsigned* nz, int rows) {
+  const int x = blockIdx.x * 64 + (threadIdx.x & 63);
+  const int y0 = blockIdx.y * 4 * rows + (threadIdx.x >> 6);
+  unsigned count = 0;
+  for (int i = 0; i < rows; ++i) {
+    const int y = y0 + 4 * i;
+    bool valid = false;
+    if (x < w && y < h) {
+      const uint8_t m = mask[(size_t)y * mpitch + x];
+      valid = m != 0;
+      const float* sp = src + (size_t)y * spitch + (size_t)x * CN;
+      float* dp = img + ((size_t)y * w + x) * CN;
+      float v[CN];
+      for (int c = 0; c < CN; ++c) v[c] = sp[c];
+      for (int c = 0; c < CN; ++c) dp[c] = valid ? v[c] : 0.f;
+      msk[(size_t)y * w + x] = (float)m * (float)(1.0 / 255.0);
+    }
+    count += (unsigned)__popcll(__ballot(valid));
   }
-  const unsigned long long b = __ballot(valid);
-  if ((threadIdx.x & 63) == 0 && b) atomicAdd(nz, (unsigned)__popcll(b));
+  apr_count(count, nz);
 }
 
 // filter2 of level l evaluated at the points downstrike_even keeps, (min(2x+1, w-1),
 // min(2y+1, h-1)) (downstrike.cc:34-75), written as level l+1; counts its non-zero mask
 template <int CN>
 __global__ void __launch_bounds__(256) k_apr_down(const float* img, const float* msk, int w, int h, float* dimg,
-                                                   float* dmsk, int dw, int dh, unsigned* nz) {
-  const int x = blockIdx.x * 64 + (threadIdx.x & 63), y = blockIdx.y * 4 + (threadIdx.x >> 6);
-  bool valid = false;
-  if (x < dw && y < dh) {
-    const int sx = min(2 * x + 1, w - 1), sy = min(2 * y + 1, h - 1);
-    double b[CN];
-    double bm = 0;
-    for (int c = 0; c < CN; ++c) b[c] = 0;
-    const float fm = msk[(size_t)sy * w + sx];
-    if (fm == 0.f) {
-      for (int dy = -1; dy <= 1; ++dy) {
-        const int r = min(max(sy + dy, 0), h - 1);
-        for (int dx = -1; dx <= 1; ++dx) {
-          const int q = min(max(sx + dx, 0), w - 1);
-          const size_t o = (size_t)r * w + q;
-          for (int c = 0; c < CN; ++c) b[c] += (double)img[o * CN + c];
-          bm += (double)msk[o];
+                                                   float* dmsk, int dw, int dh, unsigned* nz, int rows) {
+  const int x = blockIdx.x * 64 + (threadIdx.x & 63);
+  const int y0 = blockIdx.y * 4 * rows + (threadIdx.x >> 6);
+  unsigned count = 0;
+  for (int i = 0; i < rows; ++i) {
+    const int y = y0 + 4 * i;
+    bool valid = false;
+    if (x < dw && y < dh) {
+      const int sx = min(2 * x + 1, w - 1), sy = min(2 * y + 1, h - 1);
+      double b[CN];
+      double bm = 0;
+      for (int c = 0; c < CN; ++c) b[c] = 0;
+      const float fm = msk[(size_t)sy * w + sx];
+      if (fm == 0.f) {
+        for (int dy = -1; dy <= 1; ++dy) {
+          const int r = min(max(sy + dy, 0), h - 1);
+          for (int dx = -1; dx <= 1; ++dx) {
+            const int q = min(max(sx + dx, 0), w - 1);
+            const size_t o = (size_t)r * w + q;
+            for (int c = 0; c < CN; ++c) b[c] += (double)img[o * CN + c];
+            bm += (double)msk[o];
+          }
         }
       }
+      float out[CN];
+      const float om = apr_rule<CN>(fm, img + ((size_t)sy * w + sx) * CN, b, bm, out);
+      float* dp = dimg + ((size_t)y * dw + x) * CN;
+      for (int c = 0; c < CN; ++c) dp[c] = out[c];
+      dmsk[(size_t)y * dw + x] = om;
+      valid = om != 0.f;
     }
-    float out[CN];
-    const float om = apr_rule<CN>(fm, img + ((size_t)sy * w + sx) * CN, b, bm, out);
-    float* dp = dimg + ((size_t)y * dw + x) * CN;
-    for (int c = 0; c < CN; ++c) dp[c] = out[c];
-    dmsk[(size_t)y * dw + x] = om;
-    valid = om != 0.f;
+    count += (unsigned)__popcll(__ballot(valid));
   }
-  const unsigned long long bb = __ballot(valid);
-  if ((threadIdx.x & 63) == 0 && bb) atomicAdd(nz, (unsigned)__popcll(bb));
+  apr_count(count, nz);
 }
 
 // upject_even of level l+1 to the size of level l (values and the zmask of ones at the
@@ -275,23 +301,28 @@ __global__ void __launch_bounds__(256) k_apr_mask_out(const float* msk, int w, i
 
 }  // namespace
 
+// rows per thread of a level: at most 16, and 1024 blocks of the chip's 256 CUs where the level has them
+static int apr_rows(int w, int h) { return std::clamp((w + 63) / 64 * ((h + 3) / 4) / 1024, 1, 16); }
+
 hipError_t launch_apr_init(const float* src, int spitch, const uint8_t* mask, int mpitch, int w, int h, int cn,
                            float* img, float* msk, unsigned* nz, hipStream_t s) {
-  const dim3 g((w + 63) / 64, (h + 3) / 4);
+  const int rows = apr_rows(w, h);
+  const dim3 g((w + 63) / 64, (h + 4 * rows - 1) / (4 * rows));
   if (cn == 3)
-    hipLaunchKernelGGL(k_apr_init<3>, g, dim3(256), 0, s, src, spitch, mask, mpitch, w, h, img, msk, nz);
+    hipLaunchKernelGGL(k_apr_init<3>, g, dim3(256), 0, s, src, spitch, mask, mpitch, w, h, img, msk, nz, rows);
   else
-    hipLaunchKernelGGL(k_apr_init<1>, g, dim3(256), 0, s, src, spitch, mask, mpitch, w, h, img, msk, nz);
+    hipLaunchKernelGGL(k_apr_init<1>, g, dim3(256), 0, s, src, spitch, mask, mpitch, w, h, img, msk, nz, rows);
   return hipGetLastError();
 }
 
 hipError_t launch_apr_down(const float* img, const float* msk, int w, int h, int cn, float* dimg, float* dmsk, int dw,
                            int dh, unsigned* nz, hipStream_t s) {
-  const dim3 g((dw + 63) / 64, (dh + 3) / 4);
+  const int rows = apr_rows(dw, dh);
+  const dim3 g((dw + 63) / 64, (dh + 4 * rows - 1) / (4 * rows));
   if (cn == 3)
-    hipLaunchKernelGGL(k_apr_down<3>, g, dim3(256), 0, s, img, msk, w, h, dimg, dmsk, dw, dh, nz);
+    hipLaunchKernelGGL(k_apr_down<3>, g, dim3(256), 0, s, img, msk, w, h, dimg, dmsk, dw, dh, nz, rows);
   else
-    hipLaunchKernelGGL(k_apr_down<1>, g, dim3(256), 0, s, img, msk, w, h, dimg, dmsk, dw, dh, nz);
+    hipLaunchKernelGGL(k_apr_down<1>, g, dim3(256), 0, s, img, msk, w, h, dimg, dmsk, dw, dh, nz, rows);
   return hipGetLastError();
 }
 
