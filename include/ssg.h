@@ -690,6 +690,15 @@ int ssg_average_pyramid_inpaint(const ssg_image *src, const ssg_image *mask, ssg
  * src, dst: SSG_32FC1 or SSG_32FC3 of one size, host or device (dst may be src). */
 int ssg_unsharp_mask(const ssg_image *src, ssg_image *dst, double sigma, double alpha);
 
+/* ssg_inpaint_linear, ssg_average_pyramid_inpaint and ssg_unsharp_mask keep their device memory and
+ * streams for later calls: at most 2 GiB over all devices, the least recently used freed first, and
+ * given up when an allocation of the library fails.  Only memory is kept, never contents; each call in
+ * flight has its own, so calls may run on several threads.
+ * kept: bytes held now; allocations: device allocations made for such calls so far (either may be NULL). */
+int ssg_call_memory_info(uint64_t *kept, uint64_t *allocations);
+/* Frees what is held (calls in flight keep theirs). */
+int ssg_release_call_memory(void);
+
 #ifdef __cplusplus
 }
 #endif

@@ -29,7 +29,8 @@ log = logging.getLogger("serstacker_amd")
 
 __all__ = ["c_image_registration_options", "c_frame_registration", "c_weigthed_average", "image_view",
            "c_eccflow", "synth_params", "synth_render", "SsgError", "c_ser_reader", "debayer", "read_input_frames",
-           "inpaint_linear", "average_pyramid_inpaint", "unsharp_mask", "local_variance_map", "upscale_size",
+           "inpaint_linear", "average_pyramid_inpaint", "unsharp_mask", "call_memory_info",
+           "release_call_memory", "local_variance_map", "upscale_size",
            "upscale_remaps", "upscale_images",
            "master_frame_quality", "master_scan_window", "select_master_frame", "master_stack_window",
            "ecc_normalize", "focus_stack_batch"]
@@ -906,4 +907,17 @@ def unsharp_mask(src, sigma: float, alpha: float, out=None):
     sv, ov = image_view(src), image_view(out, out=True)
     _lib.check(_lib.load().ssg_unsharp_mask(C.byref(sv), C.byref(ov), sigma, alpha), "unsharp_mask")
     return out
+
+
+def call_memory_info():
+    """(bytes, allocations): the device memory that the calls without a handle keep for later calls, and the device
+    allocations made for such calls so far."""
+    kept, allocations = C.c_uint64(), C.c_uint64()
+    _lib.check(_lib.load().ssg_call_memory_info(C.byref(kept), C.byref(allocations)), "call_memory_info")
+    return kept.value, allocations.value
+
+
+def release_call_memory():
+    """Frees the device memory that the calls without a handle keep."""
+    _lib.check(_lib.load().ssg_release_call_memory(), "release_call_memory")
 

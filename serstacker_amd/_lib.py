@@ -236,6 +236,8 @@ _SIGS = [
     ("ssg_debayer", C.c_int, [_P(Image), C.c_int32, C.c_int32, _P(Image)]),
     ("ssg_inpaint_linear", C.c_int, [_P(Image), _P(Image)]),
     ("ssg_unsharp_mask", C.c_int, [_P(Image), _P(Image), C.c_double, C.c_double]),
+    ("ssg_call_memory_info", C.c_int, [_P(C.c_uint64), _P(C.c_uint64)]),
+    ("ssg_release_call_memory", C.c_int, []),
     ("ssg_average_pyramid_inpaint", C.c_int, [_P(Image), _P(Image), _P(Image), _P(Image), C.c_int32]),
     ("ssg_upscale_size", C.c_int, [C.c_int32, C.c_int32, C.c_int32, _P(C.c_int32), _P(C.c_int32)]),
     ("ssg_upscale_remaps", C.c_int, [C.c_int32, C.c_int32, _P(Image), _P(Image)]),

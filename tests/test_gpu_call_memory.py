@@ -1,0 +1,96 @@
+"""The device memory that inpainting and unsharp masking keep for later calls: a second pass allocates nothing, what
+is kept is bounded and given back, kept blocks hold nothing that a later call can see, and calls on several threads
+do not share any.  (A pass of both that allocated its planes anew took 2.3 to 11 ms for 0.46 ms of kernels.)"""
+import threading
+
+import numpy as np
+import pytest
+
+from oracle import finish as F
+
+pytestmark = pytest.mark.gpu
+
+KEEP = 2 << 30
+
+
+def _case(h, w, cn, seed):
+    rng = np.random.default_rng(seed)
+    img = rng.random((h, w, cn) if cn > 1 else (h, w)).astype(np.float32)
+    mask = np.where(rng.random((h, w)) < 0.02, 0, 255).astype(np.uint8)
+    mask[: h // 20] = 0
+    return img, mask
+
+
+def _finish(img, mask, sigma=3.0):
+    import serstacker_amd as S
+
+    full, valid = S.average_pyramid_inpaint(img, mask)
+    lin = S.inpaint_linear(img.copy(), mask)
+    return full, valid, lin, S.unsharp_mask(full, sigma, 0.6)
+
+
+def test_second_pass_allocates_nothing(oracle32):
+    import torch  # noqa: F401
+
+    import serstacker_amd as S
+
+    sizes = [(120, 160, 1), (301, 257, 3), (64, 33, 3)]
+    for k, (h, w, cn) in enumerate(sizes):
+        _finish(*_case(h, w, cn, k))
+    before = S.call_memory_info()[1]
+    for k, (h, w, cn) in enumerate(sizes):
+        img, mask = _case(h, w, cn, 10 + k)  # other contents and other buffers
+        full, valid, lin, sharp = _finish(img, mask)
+        want, want_valid = F.average_pyramid_inpaint(img, mask)
+        np.testing.assert_array_equal(full, want)
+        np.testing.assert_array_equal(valid, want_valid)
+        np.testing.assert_array_equal(sharp, F.unsharp_mask(oracle32, want, 3.0, 0.6))
+    assert S.call_memory_info()[1] == before
+
+
+def test_kept_memory_is_bounded_and_given_back():
+    import torch
+
+    import serstacker_amd as S
+
+    img = torch.rand((6000, 6000, 3), device="cuda")  # seven planes of 432 MB
+    out = torch.empty_like(img)
+    torch.cuda.synchronize()
+    for _ in range(2):
+        S.unsharp_mask(img, 1.0, 0.5, out=out)
+        assert 0 < S.call_memory_info()[0] <= KEEP
+    S.release_call_memory()
+    assert S.call_memory_info()[0] == 0
+    img, mask = _case(90, 70, 3, 5)
+    want, _ = F.average_pyramid_inpaint(img, mask)
+    np.testing.assert_array_equal(S.average_pyramid_inpaint(img, mask)[0], want)
+    assert S.call_memory_info()[0] > 0
+
+
+def test_threads_do_not_share_memory():
+    import torch  # noqa: F401
+
+    import serstacker_amd as S
+
+    cases = [_case(240 + 31 * k, 320 - 17 * k, 1 if k % 2 else 3, k) for k in range(4)]
+    want = [_finish(*c) for c in cases]
+    got, errors = [[] for _ in cases], []
+
+    def run(k):
+        try:
+            for _ in range(6):
+                got[k].append(_finish(*cases[k]))
+        except Exception as e:  # noqa: BLE001
+            errors.append(e)
+
+    threads = [threading.Thread(target=run, args=(k,)) for k in range(len(cases))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+    for k in range(len(cases)):
+        for r in got[k]:
+            for x, y in zip(r, want[k]):
+                np.testing.assert_array_equal(x, y)
+    assert S.call_memory_info()[0] <= KEEP
