@@ -2633,8 +2633,8 @@ int bayer_batch(ssg_accumulation* a, int n, const ssg_image* frames, const ssg_r
   g.valid = a->valid.as<int>();
   g.nframes = n;
   g.st = a->bayer_state();
-  // staged tiles: units of 16 or 4 bytes that every frame's rows are made of, 31-bit offsets, and a cell
-  // of one R, its diagonal B and two G
+  // staged tiles: units of 16 or 4 bytes that every frame's rows are made of, 31-bit offsets, a cell of one R,
+  // its diagonal B and two G, and maps that stay in the box
   const auto channel = [&](int q) { return (int)(a->pattern >> (2 * q) & 3u); };
   for (int q = 0; q < 4; ++q)
     if (channel(q) == 2 && channel(q ^ 3) == 0 && channel(q ^ 1) == 1 && channel(q ^ 2) == 1) {
@@ -2643,6 +2643,12 @@ int bayer_batch(ssg_accumulation* a, int n, const ssg_image* frames, const ssg_r
       for (int f = 0; f < n; ++f) bits |= (uintptr_t)ptrs[f];
       g.unit = (uint64_t)frames[0].step * a->h >= (1ull << 31) ? 0 : bits % 16 == 0 ? 16 : bits % 4 == 0 ? 4 : 0;
     }
+  for (int f = 0; f < n && g.unit; ++f)
+    if (valid[f] && !bayer_box_fits(motion_type, maps[f], a->w, a->h, type == SSG_16UC1, g.unit)) g.unit = 0;
+  // the staged kernel reads and writes the state with fewer loads in flight, which takes a few frames to make up for
+  // (4096x3000: 242 : 202 us for one frame, 263 : 225, 291 : 282, 319 : 341 for four; 1500x1000: 52 : 48, 56 : 54,
+  // 61 : 65 for three)
+  if (nvalid < (a->plane > 3 << 19 ? 4 : 3)) g.unit = 0;
   a->prof.start(s);
   HIPCHK(launch_bayer_batch(motion_type, type == SSG_16UC1, g, s));
   a->prof.stop(s, SSG_PROF_ACCUMULATE);

@@ -286,7 +286,7 @@ struct BayerBatchArgs {
   const MapCoef* maps;
   const int* valid;
   int nframes;
-  int unit;                   // 16 or 4: every row of every frame starts at a multiple of so many bytes; 0: none
+  int unit;                   // staged tiles: 16 or 4, every frame's rows start at multiples of so many bytes; else 0
   int pos_r;                  // position of R in the Bayer cell ((y & 1) << 1 | (x & 1)), B diagonal to it
   BayerState st;
 };
@@ -389,6 +389,7 @@ unsigned bayer_pattern_bits(int colorid);  // 0 for a colorid that is not a Baye
 hipError_t launch_bayer_add(const BayerState& st, const void* src, int src_pitch, bool u16, float scale,
                             const float* rmap, int rmap_pitch, const uint8_t* mask, int mask_pitch,
                             const float* wts, int wts_pitch, hipStream_t s);
+bool bayer_box_fits(int motion, const MapCoef& m, int w, int h, bool u16, int unit);
 hipError_t launch_bayer_batch(int motion, bool u16, const BayerBatchArgs& a, hipStream_t s);
 hipError_t launch_bayer_compute(const BayerState& st, float* avg, int avg_pitch, uint8_t* mask, int mask_pitch,
                                 hipStream_t s);

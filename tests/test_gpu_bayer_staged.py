@@ -1,5 +1,5 @@
 """The batched Bayer accumulate's staged tiles where their rule ends: rows that are multiples of 16 bytes,
-of 4 bytes and of neither, partial tiles, every pattern, rotations that fit the staged rows and that do not,
+of 4 bytes and of neither, partial tiles, every pattern, rotations that fit the staged rows and that do not, shifts past the frame, few frames,
 whole-pixel shifts (zero weights), and more frames than a wave classifies at a time.  Bit for bit against
 the FP32 oracle's per-frame sequence."""
 import numpy as np
@@ -72,4 +72,30 @@ def test_rotations_in_and_out_of_the_box(ssg, oracle32, motion, deg):
         tx, ty = cx - (np.cos(a) * cx - np.sin(a) * cy), cy - (np.sin(a) * cx + np.cos(a) * cy)
         params.append([tx, ty, a] if motion == 1 else
                       [np.cos(a) * 1.002, -np.sin(a), tx, np.sin(a), np.cos(a) * 0.998, ty])
+    # three frames at least go to the staged kernel
     run(ssg, oracle32, w, h, 2, True, 9, motion, params, w, 0)
+    run(ssg, oracle32, w, h, 4, True, 9, motion, params * 2, w, 0)
+    run(ssg, oracle32, w, h, 4, False, 9, motion, params * 2, w, 0)
+
+
+@pytest.mark.parametrize("u16", [True, False])
+def test_one_frame_out_of_the_box(ssg, oracle32, u16):
+    """A rotation that does not fit sends its whole batch to the general kernel."""
+    r = np.random.default_rng(12)
+    params = [[r.uniform(-5, 5), r.uniform(-5, 5), np.deg2rad(d)] for d in (0.3, -0.5, 4.0, 2.9, 0.0)]
+    run(ssg, oracle32, 208, 96, 5, u16, 8, 1, params, 208, 0)
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 4])
+def test_few_frames(ssg, oracle32, n):
+    params = [[1.5 * k - 2.25, 3.0 - 1.25 * k] for k in range(n)]
+    run(ssg, oracle32, 201, 83, n, True, 10, 0, params, 208, 0)
+
+
+@pytest.mark.parametrize("u16", [True, False])
+def test_translations_beyond_tiles_and_frames(ssg, oracle32, u16):
+    """Tiles that a shift moves wholly past an edge, and frames of which nothing is left."""
+    w, h = 208, 83
+    params = [[70.5, 0.25], [-70.5, 3.0], [2.0, 20.75], [-1.5, -20.75], [130.0, -40.5], [w + 3.5, 0.0],
+              [-w - 3.5, 1.0], [0.5, h + 2.0], [0.0, -h - 2.5], [3e4, -3e4], [0.25, -0.75]]
+    run(ssg, oracle32, w, h, len(params), u16, 11, 0, params, w, 0)
