@@ -3248,7 +3248,7 @@ extern "C" int ssg_phasecorr_estimate(ssg_phasecorr* pc, int n, const ssg_image*
   hipStream_t s = pc->stream;
   const int chunks = (n + pc->chunk - 1) / pc->chunk, chunk = (n + chunks - 1) / chunks;  // of even size
   const long long per = (long long)pc->M * pc->N;
-  const int groups = pc_groups(pc->M, pc->N);
+  const int lr = pc_rows_log2(pc->M, pc->N, chunk), groups = pc->N >> lr;
   CHK(pc->plane.ensure(sizeof(float2) * pc_plane(pc->M, pc->N) * chunk));
   CHK(pc->pv.ensure(sizeof(float) * (size_t)groups * chunk));
   CHK(pc->pi.ensure(sizeof(int) * (size_t)groups * chunk));
@@ -3266,7 +3266,7 @@ extern "C" int ssg_phasecorr_estimate(ssg_phasecorr* pc, int n, const ssg_image*
     CHK(pc_rows(pc, f0, m, pc->frame_ptrs.as<const void*>(), type == SSG_16UC1, pitch, wide));
     HIPCHK(launch_pc_cols(pc->plane.as<float2>(), pc->ref_spec.as<float2>(), pc->tw_n.as<float2>(), pc->M, pc->N,
                           pc->bh, false, m, s));
-    HIPCHK(launch_pc_peak(pc->plane.as<float2>(), pc->tw_m.as<float2>(), pc->M, pc->N, pc->binning, m,
+    HIPCHK(launch_pc_peak(pc->plane.as<float2>(), pc->tw_m.as<float2>(), pc->M, pc->N, lr, pc->binning, m,
                           pc->pv.as<float>(), pc->pi.as<int>(), pc->out.as<double>() + 3 * f0, s));
   }
   pc->prof.stop(s, SSG_PROF_FFT);

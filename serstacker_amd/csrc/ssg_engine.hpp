@@ -441,8 +441,8 @@ hipError_t launch_resize_linear(const float* src, int sw, int sh, float* dst, in
 // FFT phase correlation (ssg_fft.hip)
 constexpr int PC_PARTS_MAX = 64;  // blocks per frame of the phase correlation's mean
 // phase correlation (ssg_fft.hip): padded sizes M, N = 4 .. 4096
-int pc_groups(int M, int N);    // peak partials per frame
 size_t pc_plane(int M, int N);  // float2 elements per frame
+int pc_rows_log2(int M, int N, int nframes);  // log2 of the rows of a block of the row transforms
 hipError_t launch_pc_mean(const void* const* frames, bool u16, int pitch, bool wide, int bw, int bh, int binning,
                           float* mean, double* part, int nframes, hipStream_t s);
 hipError_t launch_pc_rows(const void* const* frames, bool u16, int pitch, bool wide, int bw, int bh, int binning,
@@ -450,8 +450,9 @@ hipError_t launch_pc_rows(const void* const* frames, bool u16, int pitch, bool w
                           int N, int nframes, hipStream_t s);
 hipError_t launch_pc_cols(float2* plane, float2* ref, const float2* tw_n, int M, int N, int bh, bool store_only,
                           int nframes, hipStream_t s);
-hipError_t launch_pc_peak(const float2* plane, const float2* tw_m, int M, int N, int binning, int nframes, float* pv,
-                          int* pi, double* out, hipStream_t s);
+// (1 << lr rows per block, N >> lr peak partials per frame)
+hipError_t launch_pc_peak(const float2* plane, const float2* tw_m, int M, int N, int lr, int binning, int nframes,
+                          float* pv, int* pi, double* out, hipStream_t s);
 
 // dense ECC flow (ssg_eccflow.hip)
 struct AreaGeom {  // one cv::resize INTER_AREA geometry, sw x sh -> dw x dh

@@ -507,16 +507,19 @@ int ilog2(int n) {
   return l;
 }
 
-// columns of a strip: 16384 points (128 KB of LDS) at the most, at most 64 columns (512-B runs)
-int strip_log2(int M, int N) { return std::min({6, ilog2(M) - 1, std::max(1, 14 - ilog2(N))}); }
-
-// log2 of the rows of a block: 8192 complex points at the most (64 KB of LDS, two blocks per CU), at most 32
-// rows, and no more than the plane has
-int rows_log2(int M, int N) { return std::min({5, 13 - ilog2(M), ilog2(N)}); }
+// log2 of the columns of a strip: 8 (64-B runs), but at most 16384 points (128 KB of LDS).  A frame's blocks are its
+// strips, so short ones are what fills the chip where the planes are small: strips of 16384 points at every size
+// (64 columns of 256 rows) were two blocks of a 256 x 256 plane, 39 us for two frames of 451 x 344 binned by 2, a call
+// of 131 us; now 89 us (95 with one row per block in memory, as before the strips).  1024 x 1024: 16 frames 319 -> 292 us.
+int strip_log2(int M, int N) { return std::min({3, ilog2(M) - 1, std::max(1, 14 - ilog2(N))}); }
 
 size_t tw_size(int n) { return n > 4 ? (size_t)n / 4 * 3 : (size_t)n / 2; }  // TW_SIZE
 
-int threads_for(int points) { return std::max(64, (points / FFT_PPT + 63) / 64 * 64); }
+// a radix-8 group per thread where the block is small (fewer rounds between two barriers), else two
+int threads_for(int points, int most) {
+  const int per = points < 8192 && points / 8 <= most ? 8 : FFT_PPT;
+  return std::max(64, (points / per + 63) / 64 * 64);
+}
 
 template <class F>
 hipError_t allow_lds(F f, size_t bytes) {
@@ -538,7 +541,13 @@ hipError_t by_log2(int l, F f) {
 
 }  // namespace
 
-int pc_groups(int M, int N) { return N >> rows_log2(M, N); }
+// 8192 complex points at the most (64 KB of LDS, two blocks per CU), at most 32 rows, and no more than the plane
+// has; down to 4 rows while the launch is below two blocks per CU
+int pc_rows_log2(int M, int N, int nframes) {
+  int lr = std::min({5, 13 - ilog2(M), ilog2(N)});
+  while (lr > 2 && (long long)nframes * (N >> lr) < 512) --lr;
+  return lr;
+}
 size_t pc_plane(int M, int N) { return 2 * (size_t)N * (M / 2 + 1); }
 
 hipError_t launch_pc_mean(const void* const* frames, bool u16, int pitch, bool wide, int bw, int bh, int binning,
@@ -553,13 +562,13 @@ hipError_t launch_pc_rows(const void* const* frames, bool u16, int pitch, bool w
                           const float* mean, const float* wx, const float* wy, const float2* tw_m, float2* plane, int M,
                           int N, int nframes, hipStream_t s) {
   const PcSource src{frames, pitch, u16 ? 1 : 0, binning, wide ? 1 : 0, bw, bh};
-  const int lr = rows_log2(M, N), lc = strip_log2(M, N);
+  const int lr = pc_rows_log2(M, N, nframes), lc = strip_log2(M, N);
   const dim3 grid((bh + (1 << lr) - 1) >> lr, nframes);
   const size_t lds = sizeof(float2) * (tw_size(M) + ((size_t)M << lr));
   return by_log2(ilog2(M), [&](auto l) {
     const hipError_t e = allow_lds(k_pc_rows<decltype(l)::value>, lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_pc_rows<decltype(l)::value>, grid, dim3(threads_for(M << lr)), lds, s, src, mean, wx, wy, tw_m,
+    hipLaunchKernelGGL(k_pc_rows<decltype(l)::value>, grid, dim3(threads_for(M << lr, 512)), lds, s, src, mean, wx, wy, tw_m,
                        plane, N, lc, lr);
     return hipGetLastError();
   });
@@ -572,24 +581,24 @@ hipError_t launch_pc_cols(float2* plane, float2* ref, const float2* tw_n, int M,
   return by_log2(ilog2(N), [&](auto l) {
     const hipError_t e = allow_lds(k_pc_cols<decltype(l)::value>, lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_pc_cols<decltype(l)::value>, dim3(nframes, ((M / 2) >> lc) + 1), dim3(threads_for(N << lc)), lds,
+    hipLaunchKernelGGL(k_pc_cols<decltype(l)::value>, dim3(nframes, ((M / 2) >> lc) + 1), dim3(threads_for(N << lc, 1024)), lds,
                        s, plane, ref, tw_n, M, lc, bh, store_only ? 1 : 0);
     return hipGetLastError();
   });
 }
 
-hipError_t launch_pc_peak(const float2* plane, const float2* tw_m, int M, int N, int binning, int nframes, float* pv,
-                          int* pi, double* out, hipStream_t s) {
-  const int lr = rows_log2(M, N), lc = strip_log2(M, N), groups = pc_groups(M, N);
+hipError_t launch_pc_peak(const float2* plane, const float2* tw_m, int M, int N, int lr, int binning, int nframes,
+                          float* pv, int* pi, double* out, hipStream_t s) {
+  const int lc = strip_log2(M, N), groups = N >> lr;
   const size_t lds = sizeof(float2) * (tw_size(M) + ((size_t)M << lr));
   const size_t lds3 = sizeof(float2) * (tw_size(M) + 3 * (size_t)M);
   return by_log2(ilog2(M), [&](auto l) {
     hipError_t e = allow_lds(k_pc_rows_peak<decltype(l)::value>, lds);
     if (e == hipSuccess) e = allow_lds(k_pc_peak<decltype(l)::value>, lds3);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_pc_rows_peak<decltype(l)::value>, dim3(groups, nframes), dim3(threads_for(M << lr)), lds, s,
+    hipLaunchKernelGGL(k_pc_rows_peak<decltype(l)::value>, dim3(groups, nframes), dim3(threads_for(M << lr, 512)), lds, s,
                        plane, tw_m, N, lc, lr, pv, pi);
-    hipLaunchKernelGGL(k_pc_peak<decltype(l)::value>, dim3(nframes), dim3(threads_for(3 * M)), lds3, s, plane, tw_m, N, lc,
+    hipLaunchKernelGGL(k_pc_peak<decltype(l)::value>, dim3(nframes), dim3(threads_for(3 * M, 768)), lds3, s, plane, tw_m, N, lc,
                        groups, binning, pv, pi, out);
     return hipGetLastError();
   });

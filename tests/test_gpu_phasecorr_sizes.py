@@ -1,5 +1,5 @@
 """The phase correlation's half-plane transforms at the sizes where their plans change (4-point axes, one
-pass of radix 4, radix 8 then 4, whole strips of 2 to 64 columns, one row pair per block) and on the
+pass of radix 4, radix 8 then 4, whole strips of 2 to 8 columns, 2 to 32 rows per block) and on the
 sources their loads treat apart (odd sizes, odd pitches, unaligned rows), against the float64 oracle."""
 import numpy as np
 import pytest
@@ -82,3 +82,19 @@ def test_unaligned_rows_give_the_aligned_rows_results(ssg, u16, binning):
         assert np.array_equal(p.estimate(views), want), (pitch, first)
     flat = torch.full((h, w), 7, dtype=torch.int16 if u16 else torch.float32, device="cuda")
     assert np.array_equal(p.estimate([flat]), np.zeros((1, 3)))
+
+
+@pytest.mark.parametrize("w,h,n", [(33, 17, 131), (250, 250, 67), (129, 513, 20), (600, 70, 9)])
+def test_any_number_of_frames_gives_the_single_frames_results(ssg, w, h, n):
+    """More frames than a launch takes (64; the last of the even-sized chunks is shorter) and launches whose blocks hold
+    4 to 32 rows by their number of frames: bit for bit the estimates of the frames one by one, also when a later call
+    has fewer frames than the planes hold."""
+    import torch
+
+    fr = [torch.from_numpy(f).cuda() for f in frames_of(w, h, n, seed=n)]
+    p = ssg.phase_correlation(w, h, 1)
+    p.set_reference(fr[0])
+    one = np.concatenate([p.estimate([f]) for f in fr[1:]])
+    assert len({tuple(o) for o in one}) > n // 2
+    for m in (n, n - 3, 5, n):
+        assert np.array_equal(p.estimate(fr[1:1 + m]), one[:m]), m
