@@ -552,9 +552,14 @@ size_t pc_plane(int M, int N) { return 2 * (size_t)N * (M / 2 + 1); }
 
 hipError_t launch_pc_mean(const void* const* frames, bool u16, int pitch, bool wide, int bw, int bh, int binning,
                           float* mean, double* part, int nframes, hipStream_t s) {
-  const PcSource src{frames, pitch, u16 ? 1 : 0, binning, wide ? 1 : 0, bw, bh};
-  hipLaunchKernelGGL(k_pc_mean_part, dim3(PC_PARTS, nframes), dim3(256), 0, s, src, part);
-  hipLaunchKernelGGL(k_pc_mean_fin, dim3(nframes), dim3(64), 0, s, part, bw, bh, mean);
+  constexpr int MOST = 32768;  // frames per launch: a grid's second dimension ends at 65535
+  for (int f0 = 0; f0 < nframes; f0 += MOST) {
+    const int n = std::min(MOST, nframes - f0);
+    const PcSource src{frames + f0, pitch, u16 ? 1 : 0, binning, wide ? 1 : 0, bw, bh};
+    double* p = part + (size_t)PC_PARTS * f0;
+    hipLaunchKernelGGL(k_pc_mean_part, dim3(PC_PARTS, n), dim3(256), 0, s, src, p);
+    hipLaunchKernelGGL(k_pc_mean_fin, dim3(n), dim3(64), 0, s, p, bw, bh, mean + f0);
+  }
   return hipGetLastError();
 }
 

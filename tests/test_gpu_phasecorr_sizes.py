@@ -98,3 +98,17 @@ def test_any_number_of_frames_gives_the_single_frames_results(ssg, w, h, n):
     assert len({tuple(o) for o in one}) > n // 2
     for m in (n, n - 3, 5, n):
         assert np.array_equal(p.estimate(fr[1:1 + m]), one[:m]), m
+
+
+def test_more_frames_than_a_grid_dimension(ssg):
+    """70000 frames (a launch's second dimension ends at 65535): every result is its frame's own."""
+    import torch
+
+    w, h, n = 24, 20, 70000
+    fr = [torch.from_numpy(f).cuda() for f in frames_of(w, h, 5, seed=3)]
+    p = ssg.phase_correlation(w, h, 1)
+    p.set_reference(fr[0])
+    one = p.estimate(fr[1:])
+    views = [ssg.image_view(f) for f in fr[1:]]
+    at = np.arange(n) * 7 // 3 % len(views)
+    assert np.array_equal(p.estimate(ssg._lib.images([views[k] for k in at])), one[at])
