@@ -1248,8 +1248,9 @@ void account_ecc_bytes(ssg_registration* r, int n, const FrameRes* res, bool has
   const bool tfirst = r->o.motion_type != SSG_MOTION_TRANSLATION && r->o.ecc.ecch_estimate_translation_first &&
                       r->o.ecc.ecch_max_level != 0;
   {
-    // every iteration of a frame at level l reads the warped current level and the reference
-    // level once (4 + 4 B/px, +1 B/px per mask); correlation passes read both level-0 images
+    // every pass of a frame at level l (an iteration that is not solved from kept moments) reads the warped
+    // current level and the reference level once (4 + 4 B/px, +1 B/px per mask); correlation passes read both
+    // level-0 images
     const int maxit = r->o.ecc.max_iterations;
     for (int f = 0; f < n; ++f) {
       for (int p = 0; p < 2; ++p) {
@@ -1257,7 +1258,7 @@ void account_ecc_bytes(ssg_registration* r, int n, const FrameRes* res, bool has
         if (p == 1 && res[f].rejected == SSG_REG_RHO_TRANSLATION) continue;
         for (int l = 0; l < r->nlevels; ++l) {
           const double bpp = 8.0 + (has_cmask ? 1.0 : 0.0) + (r->ref_has_mask[l] ? 1.0 : 0.0);
-          const int passes = std::min(res[f].level_iters[p][l], maxit);
+          const int passes = std::min(res[f].level_iters[p][l], maxit) - res[f].level_kept[p][l];
           r->prof.add_bytes(p == 0 ? SSG_PROF_ECC_TRANSLATION : SSG_PROF_ECC_MAIN, passes * bpp * r->lw[l] * r->lh[l]);
         }
       }

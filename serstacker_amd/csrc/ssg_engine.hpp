@@ -58,6 +58,7 @@ struct JRec {
 struct FrameRes {
   int level_iters[2][MAX_LEVELS];  // [pass: 0 translation-first, 1 main][level]
   int level_failed[2][MAX_LEVELS];
+  int level_kept[2][MAX_LEVELS];   // iterations among level_iters solved from kept moments (EccMemo): no pass over the image
   int rejected;                    // 0, SSG_REG_RHO_TRANSLATION or SSG_REG_RHO
   float eps;
   double rho[2];

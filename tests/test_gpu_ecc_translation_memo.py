@@ -63,3 +63,27 @@ def test_every_step_is_the_step_of_its_position(oracle64, w, h):
             oracle64.ecc_fa_align(ref.astype(np.float32), frames[f], t, max_iterations=1, max_eps=1e-7)
             assert np.abs(np.array(t.p[:2]) - path[k + 1][f]).max() < 1e-4, (f, k)
     assert revisits > 20
+
+
+@pytest.mark.gpu
+def test_profile_counts_the_bytes_of_passes_only():
+    """register_frame ends a level's passes with its last active frame, so for one frame the pass launches are the
+    passes; iterations solved from kept moments read no image."""
+    import ctypes as C
+
+    import serstacker_amd as S
+    from serstacker_amd import _lib
+    import torch
+
+    w, h = 120, 100
+    ref, frames, _ = synth_np.frames(1, w, h, radius=0.4 * h, seed=8, shift=2.0, rot_deg=0.3, noise=0.004)
+    reg = S.c_frame_registration(S.c_image_registration_options(
+        motion_type=0, scale=1.0, eps=1e-7, ecch_max_level=1, max_iterations=40, min_rho=0.0))
+    assert reg.setup_reference_frame(np.ascontiguousarray(ref, dtype=np.float32))
+    lib, prof = _lib.load(), _lib.Profile()
+    lib.ssg_registration_set_profiling(reg._h, 1)
+    assert reg.register_frame(torch.from_numpy(np.ascontiguousarray(frames[0])).cuda())
+    lib.ssg_registration_get_profile(reg._h, C.byref(prof), 1)
+    passes = prof.launches[_lib.PROF_ECC_MAIN]
+    assert reg.status().iterations == 41 and 0 < passes < 30, passes
+    assert prof.bytes[_lib.PROF_ECC_MAIN] == passes * 8.0 * w * h
