@@ -12,7 +12,8 @@
  *    Opaque handles own their device state and are released by *_destroy.
  *  - Every call returns 0 on success or a negative SSG_E_* code; the
  *    message of the last failure on the calling thread is ssg_last_error().
- *  - Handles are single-owner and not thread-safe (as the reference classes).
+ *  - Handles are single-owner and not thread-safe (as the reference classes); an average's compute
+ *    may run on several threads while nothing is added.
  *    Each handle runs its work on its own HIP stream and calls return after
  *    the stream has finished, unless documented otherwise.
  */
@@ -691,9 +692,10 @@ int ssg_average_pyramid_inpaint(const ssg_image *src, const ssg_image *mask, ssg
 int ssg_unsharp_mask(const ssg_image *src, ssg_image *dst, double sigma, double alpha);
 
 /* ssg_inpaint_linear, ssg_average_pyramid_inpaint and ssg_unsharp_mask keep their device memory and
- * streams for later calls: at most 2 GiB over all devices, the least recently used freed first, and
- * given up when an allocation of the library fails.  Only memory is kept, never contents; each call in
- * flight has its own, so calls may run on several threads.
+ * streams for later calls, ssg_accumulation_compute the device side of host images: at most 2 GiB
+ * over all devices, the least recently used freed first, and given up when an allocation of the
+ * library fails.  Only memory is kept, never contents; each call in flight has its own, so calls may
+ * run on several threads.
  * kept: bytes held now; allocations: device allocations made for such calls so far (either may be NULL). */
 int ssg_call_memory_info(uint64_t *kept, uint64_t *allocations);
 /* Frees what is held (calls in flight keep theirs). */

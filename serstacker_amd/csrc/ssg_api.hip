@@ -49,7 +49,7 @@ int fail(int code, const char* fmt, ...) {
     if (r_ != SSG_OK) return r_; \
   } while (0)
 
-// Streams and device blocks that the calls without a handle leave for later calls.  A call takes what it
+// Streams and device blocks that calls leave for later calls (those without a handle, and compute()).  A call takes what it
 // needs for itself alone and puts it back when its stream is idle; only memory is kept, never contents.
 // Why: hipFree waits for the device and unmaps, and a fresh block is mapped and cleared anew.  Eleven planes
 // allocated and freed per pass of inpaint + unsharp mask (2880x1620 RGB, 0.46 ms of kernels) made the pass
@@ -135,7 +135,8 @@ struct DevBuf {
   }
 };
 
-// The stream and the blocks of one call (CallPool), put back when it ends, on every path, its stream idle.
+// The stream and the blocks of one call (CallPool), put back when it ends, on every path, its stream idle.  The stream
+// is the pool's or a handle's (open(stream)).
 class CallScratch {
  public:
   CallScratch() = default;
@@ -145,7 +146,7 @@ class CallScratch {
     if (!s_) return;  // no block is taken before the stream
     CallPool& P = call_pool();
     const bool idle = hipStreamSynchronize(s_) == hipSuccess;
-    bool keep = false;
+    bool keep = borrowed_;
     if (idle) {
       std::lock_guard<std::mutex> lk(P.mu);
       for (CallBlock& b : mine_) {
@@ -158,7 +159,7 @@ class CallScratch {
         P.bytes += b.n;
         b.p = nullptr;
       }
-      if (P.streams.size() < CALL_STREAMS) {
+      if (!borrowed_ && P.streams.size() < CALL_STREAMS) {
         try {
           P.streams.emplace_back(dev_, s_);
           keep = true;
@@ -171,8 +172,13 @@ class CallScratch {
     if (!keep) (void)hipStreamDestroy(s_);
     (void)call_pool_trim(CALL_KEEP);
   }
-  int open() {
+  int open(hipStream_t borrow = nullptr) {
     HIPCHK(hipGetDevice(&dev_));
+    if (borrow) {
+      s_ = borrow;
+      borrowed_ = true;
+      return SSG_OK;
+    }
     CallPool& P = call_pool();
     {
       std::lock_guard<std::mutex> lk(P.mu);
@@ -224,6 +230,7 @@ class CallScratch {
  private:
   int dev_ = 0;
   hipStream_t s_ = nullptr;
+  bool borrowed_ = false;
   std::vector<CallBlock> mine_;
 };
 
@@ -1610,7 +1617,6 @@ struct ssg_accumulation {
   long long plane = 0;
   hipStream_t stream = nullptr;
   DevBuf acc, cnt, part, part_cnt, maps, weights, valid, frame_ptrs, tmp;
-  DevBuf host_avg, host_mask;  // compute() into host images: the device side of the copies
   int accumulated = 0;
   Profiler prof;
   // c_bayer_average
@@ -2839,6 +2845,10 @@ extern "C" int ssg_accumulation_compute(ssg_accumulation* a, ssg_image* avg, ssg
   if (!a) return fail(SSG_E_INVALID_ARG, "null handle");
   if (a->accumulated < 1) return fail(SSG_E_NOT_READY, "no frames accumulated");
   hipStream_t s = a->stream;
+  // the device side of host images belongs to the call: computes of one accumulator may run at once
+  CallScratch call;
+  CHK(call.open(s));
+  CallBuf host_avg(call), host_mask(call);
   float* ap = nullptr;
   size_t apb = 0;
   uint8_t* mp = nullptr;
@@ -2854,8 +2864,8 @@ extern "C" int ssg_accumulation_compute(ssg_accumulation* a, ssg_image* avg, ssg
       apb = (size_t)avg->step;
     } else {
       apb = (size_t)a->w * 4 * ocn;
-      CHK(a->host_avg.ensure(apb * a->h));
-      ap = a->host_avg.as<float>();
+      CHK(host_avg.ensure(apb * a->h));
+      ap = host_avg.as<float>();
     }
   }
   if (mask) {
@@ -2866,8 +2876,8 @@ extern "C" int ssg_accumulation_compute(ssg_accumulation* a, ssg_image* avg, ssg
       mpb = (size_t)mask->step;
     } else {
       mpb = (size_t)a->w;
-      CHK(a->host_mask.ensure(mpb * a->h));
-      mp = a->host_mask.as<uint8_t>();
+      CHK(host_mask.ensure(mpb * a->h));
+      mp = host_mask.as<uint8_t>();
     }
   }
   if (a->bayer()) {
