@@ -3201,8 +3201,8 @@ extern "C" int ssg_phasecorr_create(int32_t width, int32_t height, int32_t binni
   HIPCHK(hipMemcpyAsync(pc->wy.p, wy.data(), sizeof(float) * wy.size(), hipMemcpyHostToDevice, pc->stream));
   HIPCHK(hipMemcpyAsync(pc->tw_m.p, tm.data(), sizeof(float2) * tm.size(), hipMemcpyHostToDevice, pc->stream));
   HIPCHK(hipMemcpyAsync(pc->tw_n.p, tn.data(), sizeof(float2) * tn.size(), hipMemcpyHostToDevice, pc->stream));
-  // frames per launch: planes of 512 MB in all (16 padded 2048 x 2048 frames; 128 MB was 20 % slower, 2 GB
-  // 2 % faster)
+  // frames per launch: planes of 512 MB in all (15 padded 2048 x 2048 frames of 33.6 MB; 128 MB was 20 % slower,
+  // 2 GB 2 % faster)
   const size_t per = pc_plane(pc->M, pc->N) * sizeof(float2);
   pc->chunk = (int)std::max<size_t>(1, std::min<size_t>(64, ((size_t)512 << 20) / per));
   CHK(pc->ref_spec.ensure(per));

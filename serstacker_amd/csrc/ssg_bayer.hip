@@ -200,7 +200,7 @@ __device__ __forceinline__ void bayer_mask(const BayerState& st, const MapCoef& 
 // fma(raw * s, scale, acc), the scale being a power of two.  A wave finds the boxes of 64 frames at a time,
 // a frame per lane.
 // What bounds it: vector operations, most of them the double-precision updates and their conversions.
-// 32 raw frames of 4096x3000: 1.16 ms; 2.16 ms with sixteen two-byte gathers in flight per thread and the
+// 32 raw frames of 4096x3000: 1.14 ms; 2.16 ms with sixteen two-byte gathers in flight per thread and the
 // channel as a lane mask over three updates per tap (k_bayer_batch).
 // EDGE: frames whose mask may drop pixels of the tile are among them (a kernel of its own code: the
 // branches around a row's update keep its loads apart)
