@@ -899,6 +899,7 @@ int run_ecc(ssg_registration* r, int n, int pass, bool has_cmask, bool plain, bo
     // first counted iteration: one pass more
     const int max_passes = r->o.ecc.max_iterations + (method == ECC_LM || method == ECC_ICLM ? 1 : 0);
     for (int it = 0; it < max_passes; ++it) {
+      a.launch = it;
       a.active_in = r->active[it & 1].as<int>();
       a.active_count_in = r->active_count[it & 1].as<int>();
       a.active_out = r->active[(it + 1) & 1].as<int>();

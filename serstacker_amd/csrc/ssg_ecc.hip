@@ -411,7 +411,7 @@ __global__ void __launch_bounds__(256) k_ecc_solve(EccPassArgs a) {
   __syncthreads();
   if (wv != 0) return;
   const double sum = ((dred[0][lane] + dred[1][lane]) + dred[2][lane]) + dred[3][lane];
-  int at = 0, kept = 0;
+  int at = 0;
   if constexpr (FULL) {
     if (lane < NM) G[0][lane] = sum;
   } else {
@@ -438,7 +438,7 @@ __global__ void __launch_bounds__(256) k_ecc_solve(EccPassArgs a) {
     ecc_solve<MOTION, FULL>(G[0], X, a.res[f], a, lane == 0);
   } else {
     // ecc_solve ends the loop at the latest when the iteration budget is spent
-    for (;; ++kept) {
+    for (;;) {
       ecc_solve<MOTION, FULL>(G[at], X, a.res[f], a, lane == 0);
       int qx, qy;
       if (!(X.flags & XF_ACTIVE) || !translation_key(X.p[0], a.w, qx) || !translation_key(X.p[1], a.h, qy)) break;
@@ -458,11 +458,13 @@ __global__ void __launch_bounds__(256) k_ecc_solve(EccPassArgs a) {
     to_xf.iters = X.iters;
     to_xf.flags = X.flags;
     to_xf.eps = X.eps;
-    if (kept) atomicAdd(&a.res[f].level_kept[a.pass][a.level], kept);  // (no load to wait for)
     if (X.flags & XF_ACTIVE) {
       // the list order does not affect any frame's result
       const int to = atomicAdd(a.active_count_out, 1);
       a.active_out[to] = f;
+    } else if constexpr (!FULL) {
+      // the frame was active in every launch of the level up to this one
+      a.res[f].level_kept[a.pass][a.level] = X.iters - (a.launch + 1);
     }
   }
 }

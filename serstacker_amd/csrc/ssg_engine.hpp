@@ -128,6 +128,7 @@ struct EccPassArgs {
   int nframes;
   int pass, level;
   int max_iterations;
+  int launch;             // of the level's passes, from 0
   float max_eps;
   double update_step_scale;
   EccMemo* memo;          // per frame, forward-additive translation passes
