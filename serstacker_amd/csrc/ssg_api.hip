@@ -2653,9 +2653,9 @@ int bayer_batch(ssg_accumulation* a, int n, const ssg_image* frames, const ssg_r
     }
   for (int f = 0; f < n && g.unit; ++f)
     if (valid[f] && !bayer_box_fits(motion_type, maps[f], a->w, a->h, type == SSG_16UC1, g.unit)) g.unit = 0;
-  // the staged kernel reads and writes the state with fewer loads in flight, which takes a few frames to make up for
-  // (4096x3000: 242 : 202 us for one frame, 263 : 225, 291 : 282, 319 : 341 for four; 1500x1000: 52 : 48, 56 : 54,
-  // 61 : 65 for three)
+  // the staged kernel reads and writes the state with fewer loads in flight, which takes a few frames to make up for:
+  // 4096x3000 staged 242, 263, 291, 319 us for one to four frames, general 202, 225, 282, 341; 1500x1000 staged
+  // 52, 56, 61 for one to three, general 48, 54, 65 (1330x1298 still 133 : 130 for three)
   if (nvalid < (a->plane > 3 << 19 ? 4 : 3)) g.unit = 0;
   a->prof.start(s);
   HIPCHK(launch_bayer_batch(motion_type, type == SSG_16UC1, g, s));
