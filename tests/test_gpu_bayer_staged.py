@@ -72,10 +72,22 @@ def test_rotations_in_and_out_of_the_box(ssg, oracle32, motion, deg):
         tx, ty = cx - (np.cos(a) * cx - np.sin(a) * cy), cy - (np.sin(a) * cx + np.cos(a) * cy)
         params.append([tx, ty, a] if motion == 1 else
                       [np.cos(a) * 1.002, -np.sin(a), tx, np.sin(a), np.cos(a) * 0.998, ty])
-    # three frames at least go to the staged kernel
     run(ssg, oracle32, w, h, 2, True, 9, motion, params, w, 0)
-    run(ssg, oracle32, w, h, 4, True, 9, motion, params * 2, w, 0)
-    run(ssg, oracle32, w, h, 4, False, 9, motion, params * 2, w, 0)
+
+
+@pytest.mark.parametrize("u16", [True, False])
+@pytest.mark.parametrize("motion", [1, 3])
+@pytest.mark.parametrize("deg", [0.5, 1.9, 2.9, 3.4, 9.0, 179.0])
+def test_rotations_of_enough_frames_for_the_staged_kernel(ssg, oracle32, u16, motion, deg):
+    w, h = 208, 160
+    params = []
+    for k, s in enumerate((1, -1, 0.9, -0.8)):
+        a = np.deg2rad(deg * s)
+        cx, cy = w / 2 + 0.3 * k, h / 2 - 0.2
+        tx, ty = cx - (np.cos(a) * cx - np.sin(a) * cy), cy - (np.sin(a) * cx + np.cos(a) * cy)
+        params.append([tx, ty, a] if motion == 1 else
+                      [np.cos(a) * 1.002, -np.sin(a), tx, np.sin(a), np.cos(a) * 0.998, ty])
+    run(ssg, oracle32, w, h, 4, u16, 9, motion, params, w, 0)
 
 
 @pytest.mark.parametrize("u16", [True, False])
